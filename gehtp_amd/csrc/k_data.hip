@@ -7,12 +7,13 @@
 // with g = r / 32, phase = (r % 32) / 4, rp = (r % 4) / 2, kt = c / 32.
 #include "kernels.h"
 
+#include <cmath>
+
 namespace gehtp {
 
 namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef short s2_t __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ size_t crouton_pos(uint32_t r, uint32_t c, uint32_t n_m32, uint32_t n_kt) {
     const uint32_t rr = r & 31u;
@@ -57,96 +58,221 @@ __global__ void crouton_decode_kernel(const uint32_t* __restrict__ surf, uint16_
 }
 
 // ---------------------------------------------------------------------------
-// OP_MATMUL_W4A16: Y[m,n] = clip(nearest((sum_k (A[m,k]-32768) W[k,n]) / 7) + 32768).
-// Workgroup tile 64 (m) x 64 (n), K step 32. A comes straight from the crouton act
-// surface: the (kt, g) 32x32 block is 16 contiguous 128-byte chunks (8 phases x 2 row
-// pairs); A - 32768 as int16 is A ^ 0x8000. W rows ([N][K/2], +8 nibbles) unpack to
-// int16 in LDS. Products accumulate with v_dot2_i32_i16 in int32 per K step (at most
-// 32 * 2^15 * 8 = 2^23) and in int64 across steps. Results go to the crouton out surface.
-constexpr int WA_BM = 64, WA_BN = 64, WA_BK = 32, WA_LD = WA_BK + 2;   // int16 row stride (pairs stay aligned)
+// OP_MATMUL_W4A16: Y[m,n] = clip(nearest((sum_k (A[m,k]-32768) W[k,n]) / 7) + 32768), in
+// whole numbers on the matrix cores (v_mfma_i32_32x32x32_i8). A u16 activation is two
+// signed bytes once its bytes' top bits are flipped (word ^ 0x80808080): A - 32768 =
+// 256 hi + lo + 128, so the sum is 256 sum(hi W) + sum(lo W) + 128 sum(W), the last from
+// v_dot4 on the weight words. A stored nibble (q + 8) ^ 8 is q in two's complement; left in
+// a byte's top half it is 16 q, so 8 weights unpack with a shift and two xor-ands (even k's
+// in one word, odd ones in the other; A's columns are staged in that order), and the sums,
+// all multiples of 16, are shifted down exactly.
+// Workgroup tile 32 RT x 32 NT, its K steps (64 = two 32-column blocks of the surface)
+// split over 8 waves in contiguous ranges: at these sizes (M = 256, K = N = 2560: 160 tiles
+// of 64 x 64) a serial K loop is latency. Each wave stages its own A block in LDS
+// (256 RT-byte runs of the surface in, byte planes out), so its loop needs no barrier; W
+// goes from memory to the B operand. The waves' sums meet in LDS. int32 holds the tile's
+// whole sums up to 8064 columns (8064 * 32896 * 8 < 2^31); longer K runs in such chunks with
+// int64 totals between them.
+// Bound: no one unit. Counters at 1024 x 4096 x 4096 (64 x 64 tiles): VALU issue 51 % of the
+// CU's cycles (the byte planes: 24 instructions per 16 u16 pairs), LDS 41 %, L1 55 %, MFMA
+// 24 %. 256 x 2560 x 2560: 134.9 -> 12.5 us per call (the 64 x 64 v_dot2 tiles it replaces, one wave
+// row per 16 columns and a barrier per 32 columns, against this).
+constexpr uint32_t WA_WV = 8;
+constexpr uint32_t kWaChunk = 126;   // K steps of an int32 chunk: 8064 columns
 
-__device__ __forceinline__ int64_t round_div7(int64_t s) { return s >= 0 ? (s + 3) / 7 : -((-s + 3) / 7); }
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32_a2 __attribute__((aligned(2)));   // surfaces need only be u16-aligned on output
 
-__global__ __launch_bounds__(256) void w4a16_gemm_kernel(const uint16_t* __restrict__ act,
-                                                         const uint8_t* __restrict__ w,
-                                                         uint16_t* __restrict__ out, uint32_t M,
-                                                         uint32_t K, uint32_t N) {
-    __shared__ __align__(16) int16_t As[WA_BM * WA_LD];
-    __shared__ __align__(16) int16_t Ws[WA_BN * WA_LD];
-    const uint32_t tid = threadIdx.x;
-    const uint32_t m0 = blockIdx.y * WA_BM, n0 = blockIdx.x * WA_BN;
-    const uint32_t n_m32 = M >> 5, n_kt = K >> 5;
-    const uint32_t tm = tid >> 4, tn = tid & 15;   // 4 x 4 outputs: rows tm*4.., cols tn*4..
-    int64_t tot[4][4];
+template <typename T>   // nearest of s / 7 (no ties), clipped to a u16 around the zero point
+__device__ __forceinline__ uint32_t w4a16_out(T s) {
+    const T y = (s >= 0 ? (s + 3) / 7 : -((-s + 3) / 7)) + 32768;
+    return y < 0 ? 0u : y > 65535 ? 65535u : (uint32_t)y;
+}
+
+template <int RT, int NT, int MINW>
+__global__ __launch_bounds__(64 * WA_WV, MINW) void w4a16_gemm_kernel(const uint16_t* __restrict__ act,
+                                                                      const uint8_t* __restrict__ w,
+                                                                      uint16_t* __restrict__ out, uint32_t M,
+                                                                      uint32_t K, uint32_t N) {
+    // A staged plane: rows of 64 bytes at a stride of 80 (operand reads of 16 rows and
+    // stores of every second row then spread over all banks), 128 bytes between row tiles.
+    constexpr uint32_t RS = 80, TS = 32 * RS + 128, PLANE = RT * TS, NU = 2 * RT;
+    constexpr uint32_t CS = 32 * RT + 4, TILE = 32 * CS;   // a wave's sums of one n tile: [column][row], padded
+    constexpr uint32_t NQ = RT * 512 / (64 * WA_WV);       // surface words per thread and n tile
+    constexpr uint32_t WLDS = 2 * PLANE > TILE * 4 ? 2 * PLANE : TILE * 4;
+    __shared__ __align__(16) uint8_t lds[WA_WV * WLDS];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5, l32 = lane & 31;
+    const uint32_t n_m32 = M >> 5, n_kt = K >> 5, nsteps = (n_kt + 1) / 2;
+    const uint32_t nt = (N / 32 + NT - 1) / NT, g0 = (blockIdx.x / nt) * RT, n0 = (blockIdx.x % nt) * (32 * NT);
+    uint8_t* st = lds + wave * WLDS;
+
+    // A: a unit is 8 columns x one row pair (32 contiguous bytes); a phase's chunks of the
+    // tile are 256 RT contiguous bytes per block. Unit 64 i + lane = (phase, kt, group,
+    // pair, 8 columns).
+    const uint32_t urp = (lane >> 2) & 1, uoct = lane & 3;
+    const uint32_t ugl = RT == 2 ? (lane >> 3) & 1 : 0, ukt = RT == 2 ? (lane >> 4) & 1 : (lane >> 3) & 1;
+    const uint32_t uph = RT == 2 ? lane >> 5 : lane >> 4;   // + (8 / NU) i
+    const uint32_t ug = min(g0 + ugl, n_m32 - 1);           // rows past M repeat the last group (not stored)
+    const size_t kt_bytes = (size_t)n_m32 * 256, ph_bytes = kt_bytes * n_kt;
+    const uint8_t* abase = reinterpret_cast<const uint8_t*>(act) + uph * ph_bytes + (size_t)ug * 256 + urp * 128 + uoct * 32;
+    uint8_t* sta = st + ugl * TS + (uph * 4 + urp * 2) * RS + ukt * 32 + uoct * 8;
+    const uint8_t* wbase[NT];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < NT; ++j) wbase[j] = w + (size_t)min(n0 + 32 * j + l32, N - 1) * (K / 2);
+    u32x4 ra[NU][2], rw[NT];
+    auto load = [&](uint32_t s) __attribute__((always_inline)) {
+        const uint32_t kw = min(2 * s + half, n_kt - 1);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) tot[i][j] = 0;
+        for (int j = 0; j < NT; ++j) rw[j] = *reinterpret_cast<const u32x4*>(wbase[j] + kw * 16);
+        const uint8_t* p = abase + min(2 * s + ukt, n_kt - 1) * kt_bytes;
+#pragma unroll
+        for (uint32_t i = 0; i < NU; ++i) {
+            const u32x4* q = reinterpret_cast<const u32x4*>(p + i * (8 / NU) * ph_bytes);
+            ra[i][0] = q[0];
+            ra[i][1] = q[1];
+        }
+    };
 
-    for (uint32_t kt = 0; kt < n_kt; ++kt) {
-        // A: 2 row groups x 16 chunks x 8 pieces of 16 bytes = 256 pieces, one per thread.
-        {
-            const uint32_t gl = tid >> 7, u = tid & 127, ch = u >> 3, piece = u & 7;
-            const uint32_t phase = ch >> 1, rp = ch & 1;
-            const uint32_t g = (m0 >> 5) + gl;
-            if (g < n_m32) {
-                const size_t chunk = ((size_t)(phase * n_kt + kt) * n_m32 + g) * 2 + rp;
-                const u32x4 v = *reinterpret_cast<const u32x4*>(act + chunk * 64 + piece * 8);
-                const uint32_t r0 = gl * 32 + phase * 4 + rp * 2;   // local row of the pair
+    int64_t tot[NT][NQ][2];   // [n tile][word][row of the pair]
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (uint32_t e = 0; e < 2 * NQ; ++e) tot[j][e >> 1][e & 1] = 0;
+
+    for (uint32_t c0 = 0; c0 < nsteps; c0 += kWaChunk) {
+        const uint32_t cn = min(kWaChunk, nsteps - c0), per = (cn + WA_WV - 1) / WA_WV;
+        const uint32_t s0 = c0 + min(wave * per, cn), s1 = c0 + min((wave + 1) * per, cn);
+        i32x16 acc[NT][2][RT];   // [n tile][plane][row tile]
+        int wsum[NT];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            wsum[j] = 0;
+#pragma unroll
+            for (int e = 0; e < 2 * RT; ++e)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[j][e / RT][e % RT][r] = 0;
+        }
+        load(min(s0, nsteps - 1));   // loads are unconditional: a branch would drain them at its join
+#pragma unroll 1
+        for (uint32_t s = s0; s < s1; ++s) {
+            // byte planes of this step's block, and its weights, out of the load registers
+#pragma unroll
+            for (uint32_t i = 0; i < NU; ++i) {
+                const u32x4 a = ra[i][0] ^ 0x80808080u, b = ra[i][1] ^ 0x80808080u;
+                uint32_t pl[2][2][2];   // [plane][row][even / odd columns]
+#pragma unroll
+                for (int o = 0; o < 2; ++o) {
+                    const uint32_t t0 = __builtin_amdgcn_perm(a[o + 2], a[o], 0x05010400u);
+                    const uint32_t t1 = __builtin_amdgcn_perm(b[o + 2], b[o], 0x05010400u);
+                    const uint32_t t2 = __builtin_amdgcn_perm(a[o + 2], a[o], 0x07030602u);
+                    const uint32_t t3 = __builtin_amdgcn_perm(b[o + 2], b[o], 0x07030602u);
+                    pl[0][0][o] = __builtin_amdgcn_perm(t1, t0, 0x05040100u);
+                    pl[1][0][o] = __builtin_amdgcn_perm(t1, t0, 0x07060302u);
+                    pl[0][1][o] = __builtin_amdgcn_perm(t3, t2, 0x05040100u);
+                    pl[1][1][o] = __builtin_amdgcn_perm(t3, t2, 0x07060302u);
+                }
+#pragma unroll
+                for (int p = 0; p < 2; ++p)
+#pragma unroll
+                    for (int b2 = 0; b2 < 2; ++b2)
+                        *reinterpret_cast<uint64_t*>(sta + p * PLANE + (i * (32 / NU) + b2) * RS) =
+                            (uint64_t)pl[p][b2][1] << 32 | pl[p][b2][0];
+            }
+            i32x4 bop[NT][2];
+            // 0: past an odd block count, the last step's second block counts as zero weights
+            const uint32_t nib = 2 * s + half < n_kt ? 0xF0F0F0F0u : 0u;
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const uint32_t col = piece * 4 + e;
-                    const uint32_t x = v[e] ^ 0x80008000u;
-                    As[r0 * WA_LD + col] = (int16_t)(x & 0xFFFFu);
-                    As[(r0 + 1) * WA_LD + col] = (int16_t)(x >> 16);
+                    const uint32_t x = rw[j][e];
+                    const int ev = (int)(((x << 4) ^ 0x80808080u) & nib), od = (int)((x ^ 0x80808080u) & nib);
+                    bop[j][e >> 1][2 * (e & 1)] = ev;
+                    bop[j][e >> 1][2 * (e & 1) + 1] = od;
+                    wsum[j] = __builtin_amdgcn_sdot4(ev, 0x01010101, wsum[j], false);
+                    wsum[j] = __builtin_amdgcn_sdot4(od, 0x01010101, wsum[j], false);
                 }
+            load(min(s + 1, nsteps - 1));
+            __builtin_amdgcn_sched_barrier(0);
+            // the wave's lanes read what other lanes of it wrote: DS operations of a wave
+            // complete in order, the fences keep the compiler from moving them across
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int p = 0; p < 2; ++p)
+#pragma unroll
+                    for (int t = 0; t < RT; ++t) {
+                        const i32x4 av =
+                            *reinterpret_cast<const i32x4*>(st + p * PLANE + t * TS + l32 * RS + half * 32 + q * 16);
+#pragma unroll
+                        for (int j = 0; j < NT; ++j)
+                            acc[j][p][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, bop[j][q], acc[j][p][t], 0, 0, 0);
+                    }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+        // Sums over the waves, one n tile at a time: [wave][column][row]. Thread t holds
+        // surface words (row pair, column) = t, t + 512.
+        int* red = reinterpret_cast<int*>(lds);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            __syncthreads();
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; r += 4) {   // 256 hi + lo, without the factor 16
+                    i32x4 v;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = acc[j][1][t][r + e] * 16 + (acc[j][0][t][r + e] >> 4);
+                    *reinterpret_cast<i32x4*>(&red[wave * TILE + l32 * CS + t * 32 + 2 * r + 4 * half]) = v;
+                }
+            __syncthreads();
+#pragma unroll
+            for (uint32_t q = 0; q < NQ; ++q) {
+                const uint32_t idx = tid + 512 * q, col = idx & 31, pr = idx >> 5;
+                int sum[2] = {0, 0};
+#pragma unroll
+                for (uint32_t v = 0; v < WA_WV; ++v) {
+                    const int2 x = *reinterpret_cast<const int2*>(&red[v * TILE + col * CS + 2 * pr]);
+                    sum[0] += x.x;
+                    sum[1] += x.y;
+                }
+                tot[j][q][0] += sum[0];
+                tot[j][q][1] += sum[1];
             }
         }
-        // W: 64 rows x 16 bytes (32 nibbles) of this K step.
-        if (tid < WA_BN) {
-            const uint32_t n = n0 + tid;
-            u32x4 v = {0x88888888u, 0x88888888u, 0x88888888u, 0x88888888u};   // q = 0 past N
-            if (n < N) v = *reinterpret_cast<const u32x4*>(w + (size_t)n * (K / 2) + kt * 16);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int b = 0; b < 8; ++b)
-                    Ws[tid * WA_LD + e * 8 + b] = (int16_t)((int32_t)((v[e] >> (4 * b)) & 0xFu) - 8);
-        }
         __syncthreads();
-        int32_t acc[4][4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int j = 0; j < NT; ++j) red[(j * WA_WV + wave) * 64 + lane] = wsum[j] >> 4;   // this lane's k half of column l32
+        __syncthreads();
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = 0;
+        for (int j = 0; j < NT; ++j) {
+            int ws = 0;
 #pragma unroll
-        for (int kk = 0; kk < WA_BK; kk += 2) {
-            s2_t a2[4], w2[4];
+            for (uint32_t v = 0; v < 2 * WA_WV; ++v) ws += red[j * WA_WV * 64 + v * 32 + (tid & 31)];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) a2[i] = *reinterpret_cast<const s2_t*>(&As[(tm * 4 + i) * WA_LD + kk]);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) w2[j] = *reinterpret_cast<const s2_t*>(&Ws[(tn * 4 + j) * WA_LD + kk]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_sdot2(a2[i], w2[j], acc[i][j], false);
+            for (uint32_t e = 0; e < 2 * NQ; ++e) tot[j][e >> 1][e & 1] += (int64_t)ws * 128;
         }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) tot[i][j] += acc[i][j];
         __syncthreads();
     }
-    const uint32_t on_m32 = M >> 5, on_kt = N >> 5;
+
+    const uint32_t on_kt = N >> 5;
+    const bool small = nsteps <= kWaChunk;   // the whole sum fits int32
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t m = m0 + tm * 4 + i, n = n0 + tn * 4 + j;
-            if (m >= M || n >= N) continue;
-            int64_t v = round_div7(tot[i][j]) + 32768;
-            v = v < 0 ? 0 : (v > 65535 ? 65535 : v);
-            out[crouton_pos(m, n, on_m32, on_kt)] = (uint16_t)v;
+        for (uint32_t q = 0; q < NQ; ++q) {
+            const uint32_t idx = tid + 512 * q, col = idx & 31, m = g0 * 32 + 2 * (idx >> 5), kt = (n0 >> 5) + j;
+            if (m >= M || kt >= on_kt) continue;
+            uint32_t v[2];
+#pragma unroll
+            for (int b = 0; b < 2; ++b) v[b] = small ? w4a16_out((int32_t)tot[j][q][b]) : w4a16_out(tot[j][q][b]);
+            const uint32_t rr = m & 31u;
+            const size_t chunk = ((size_t)((rr >> 2) * on_kt + kt) * n_m32 + (m >> 5)) * 2 + ((rr >> 1) & 1u);
+            *reinterpret_cast<u32_a2*>(out + chunk * 64 + 2 * col) = v[0] | (v[1] << 16);
         }
 }
 
@@ -316,8 +442,24 @@ hipError_t launch_matmul_w4a16(const uint16_t* act, const uint8_t* w, uint16_t* 
                                uint32_t N, hipStream_t st) {
     if (M % 32 || K % 32 || N % 32) return hipErrorInvalidValue;
     if (!M || !N || !K) return hipSuccess;
-    hipLaunchKernelGGL(w4a16_gemm_kernel, dim3((N + WA_BN - 1) / WA_BN, (M + WA_BM - 1) / WA_BM), dim3(256), 0, st,
-                       act, w, out, M, K, N);
+    // Tile by the time of the grid's rounds. A round (one workgroup on every CU) took 5.8 us
+    // with 32 x 32 tiles (two fit a CU: 8.3 us a pair), 8.2 with 32 x 64 and 12 with 64 x 64
+    // at K = 2560, in like proportion at other K. Measured with 32 x 32 / 32 x 64 / 64 x 64
+    // tiles, us (M x N x K): 32 x 2560 x 2560 5.8 / 7.8 / 11.1; 256 x 2560 x 2560 14.7 / 16.5 /
+    // 12.6; 512 x 2560 x 2560 22.5 / 24.6 / 23.5; 1024 x 512 x 4096 17.4 / 15.4 / 18.9;
+    // 1024 x 4096 x 4096 91 / 82 / 62.
+    const size_t cus = (size_t)device_cu_count();
+    auto grid = [&](uint32_t rt, uint32_t nt) { return (size_t)((M / 32 + rt - 1) / rt) * ((N / 32 + nt - 1) / nt); };
+    auto rounds = [&](size_t g) { return (double)((g + cus - 1) / cus); };
+    const double r11 = rounds(grid(1, 1));
+    const double t11 = 8.3 * std::floor(r11 / 2) + 5.8 * std::fmod(r11, 2.0);
+    const double t12 = 8.2 * rounds(grid(1, 2)), t22 = 12.0 * rounds(grid(2, 2));
+    auto go = [&](auto kern, uint32_t rt, uint32_t nt) {
+        hipLaunchKernelGGL(kern, dim3((uint32_t)grid(rt, nt)), dim3(64 * WA_WV), 0, st, act, w, out, M, K, N);
+    };
+    if (t22 < t11 && t22 < t12) go(w4a16_gemm_kernel<2, 2, 2>, 2, 2);
+    else if (t12 < t11) go(w4a16_gemm_kernel<1, 2, 2>, 1, 2);
+    else go(w4a16_gemm_kernel<1, 1, 4>, 1, 1);
     return hipGetLastError();
 }
 

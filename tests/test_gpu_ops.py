@@ -253,3 +253,24 @@ def test_engine_data_ops(engine, oracle):
     assert np.array_equal(got("pad", pd.size), pd.view(np.uint16))
     dma = np.frombuffer(engine.temp(T["dma"]), np.uint8)[8:8 + 64]
     assert np.array_equal(dma, pd.view(np.uint8)[32:96])
+
+
+@pytest.mark.parametrize("M,K,N", [(32, 32, 96), (32, 96, 1056), (64, 8064, 64), (64, 8096, 32), (96, 544, 4064),
+                                   (256, 576, 2592), (1024, 160, 544)])
+def test_matmul_w4a16_tiles(lib, oracle, torch_dev, M, K, N):
+    """Opcode 1's tile shapes and remainders on 256 CUs: 32 x 32, 32 x 64 and 64 x 64 tiles,
+    an odd row or column tile at the edge, an odd number of 32-column blocks (the last K
+    step half empty), fewer K steps than waves, and K on both sides of the longest int32
+    chunk with every product at its largest. Whole numbers: bit for bit."""
+    import torch
+    rng = np.random.default_rng(M + K + N)
+    A = rng.integers(0, 65536, size=(M, K), dtype=np.uint16)
+    W = rng.integers(-8, 8, size=(N, K), dtype=np.int8)
+    if K > 8000:   # the largest sums either way
+        A[0], A[1], W[0], W[1] = 0, 65535, -8, 7
+    act, wslot = oracle.crouton_encode(A), oracle.w4a16_pack(W)
+    out = torch.empty(M * N, dtype=torch.int16, device=torch_dev)
+    assert lib.gehtp_matmul_w4a16(ptr(to_dev(act.view(np.int16), torch_dev)), ptr(to_dev(wslot, torch_dev)), ptr(out),
+                                  M, K, N, stream_ptr()) == 0
+    _sync()
+    assert np.array_equal(out.cpu().numpy().view(np.uint16), oracle.matmul_w4a16(act, wslot, M, K, N))
