@@ -738,3 +738,43 @@ def test_attn_decode_qkv_matches_unfused(lib, oracle, torch_dev, H, KVH, pos0):
     ring_chk.posmap[:n_kv] = np.arange(n_kv, dtype=np.uint32)
     ref = ring_chk.attn_decode(from_dev(q_b), n_kv, H, KVH, hd, SCALE)
     assert_close(from_dev(out_a), ref, what=f"decode_qkv H={H} KVH={KVH} n_kv={n_kv}")
+
+
+@pytest.mark.parametrize("M,K,N,Bn", [(1, 1024, 48, 1), (2, 2050, 33, 1), (3, 700, 9, 1), (4, 2048, 8, 2), (1, 260, 8200, 1),
+                                      (1, 3, 7, 1), (5, 7, 5, 1), (33, 128, 32, 1), (5, 641, 31, 1), (31, 1025, 45, 3),
+                                      (64, 200, 1000, 8), (65, 1022, 4100, 1), (700, 131, 1300, 1), (1000, 64, 70, 40),
+                                      (1030, 72, 8200, 1), (1030, 79, 8201, 1), (2050, 66, 4097, 2)])
+def test_matmul_f16_tiles_and_edges(lib, torch_dev, M, K, N, Bn):
+    """The tiles (32, 64 and 128 square by the grid's size; 16- and 32-column GEMV
+    workgroups), their remainders in M, N and K, rows off every alignment, rows of fewer
+    than 8 elements, every layout flag and a column window, against float32 products of the
+    same values: the result rounds to fp16 once (2^-11), and fp32 sums of K products of
+    values around 1/sqrt(K) are off by at most K 2^-24 of the sum of magnitudes. A NaN and an
+    infinity in one row of A and one column of W reach that row and column alone."""
+    import torch
+    g = torch.Generator(device=torch_dev).manual_seed(M * 31 + K * 7 + N)
+    for flags in (0, 1, 2, 3) if Bn == 1 else (4, 6):
+        for n0, pad, off in ((0, 0, 0), (5, 9, 1)):   # a column window; operands starting 2 bytes off
+            t0, t1, Nf = bool(flags & 1) and Bn == 1, bool(flags & 2), n0 + N + pad
+            a = torch.randn((Bn, M, K), device=torch_dev, generator=g).half()
+            w = (torch.randn((Bn, K, Nf), device=torch_dev, generator=g) * K ** -0.5).half()
+            if M > 1:
+                a[:, M // 2, K // 2] = float("nan")
+                w[:, K - 1, n0 + N - 1] = float("inf")
+            ab = torch.empty(a.numel() + off, dtype=torch.float16, device=torch_dev)
+            wb = torch.empty(w.numel() + off, dtype=torch.float16, device=torch_dev)
+            ab[off:] = (a.transpose(1, 2) if t0 else a).reshape(-1)
+            wb[off:] = (w.transpose(1, 2) if t1 else w).reshape(-1)
+            y = torch.full((Bn, M, Nf), 7.0, dtype=torch.float16, device=torch_dev)
+            assert lib.gehtp_matmul_f16(ab.data_ptr() + 2 * off, wb.data_ptr() + 2 * off, ptr(y), M, K, Nf, n0, N,
+                                        flags | (Bn << 16), stream_ptr()) == 0
+            _sync()
+            win, what = y[:, :, n0:n0 + N].double(), f"{M}x{K}x{N} b{Bn} f{flags} n0={n0}"
+            assert (y[:, :, :n0] == 7).all() and (y[:, :, n0 + N:] == 7).all(), what
+            ref = torch.stack([a[b].double() @ w[b, :, n0:n0 + N].double() for b in range(Bn)])
+            mag = torch.stack([a[b].double().abs() @ w[b, :, n0:n0 + N].double().abs() for b in range(Bn)])
+            ok = torch.isfinite(ref)
+            assert torch.equal(torch.isnan(win), torch.isnan(ref)) and torch.equal(win[~ok & ~torch.isnan(ref)],
+                                                                                   ref[~ok & ~torch.isnan(ref)]), what
+            err = (win - ref)[ok].abs()
+            assert (err <= ref[ok].abs() * 2 ** -11 + mag[ok] * K * 2 ** -24 + 2 ** -24).all(), (what, float(err.max()))
