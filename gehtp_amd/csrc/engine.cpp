@@ -1192,9 +1192,11 @@ int op_w4g_fused(Ctx& cx) {
     // The OP_QK_ROPE_KV_F16 that reads this q|k|v output next, in the same run: the
     // GEMM's epilogue performs it (after a table kernel that fixes the positions and
     // advances the counter), writing y as well, and that op then finds its work done.
-    // Shapes or operands the epilogue cannot take leave the op to run (or fail) alone.
+    // Shapes or operands the epilogue cannot take leave the op to run (or fail) alone, and so
+    // do few rows, whose GEMM is another kernel (M = 8, N 4096, K 1024: 3.4 us and the op's 4,
+    // against 6.8 and the table's 4).
     const wt_op* rx = cx.op + 1;
-    if (fusion_on() && !swiglu && !res && ldy == N && (uint32_t)(rx - cx.b->ops) < g_run_end &&
+    if (fusion_on() && !w4g_gemm_skinny(M) && !swiglu && !res && ldy == N && (uint32_t)(rx - cx.b->ops) < g_run_end &&
         rx->opcode == OP_QK_ROPE_KV_F16 && rx->n_args >= 12 && rx->args[0] == A(3) && rx->args[5] == M &&
         rx->args[8] == 128 && (uint64_t)(rx->args[6] + 2ull * rx->args[7]) * 128u == N) {
         QkRope r;

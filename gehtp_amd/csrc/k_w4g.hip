@@ -19,6 +19,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <type_traits>
 
 namespace gehtp {
 
@@ -701,6 +702,155 @@ __global__ __launch_bounds__(256, 3) void w4g_gemm_kernel(
     w4g_plain_tiles(acc, lane, m0, n0 + wn * 32 * WJ, M, N, y, ldy, res, ldr, part, split);
 }
 
+// ---------------------------------------------------------------------------
+// GEMM of few rows (M <= 32): weights stream once, so a tile is 16 NT columns of all M rows
+// (AR >= M of them staged) and K is split over the workgroup's WV waves in contiguous ranges
+// of 128-deep blocks, their sums added in LDS in wave order; no workspace, one launch. On
+// v_mfma_f32_16x16x32_f16 lane l supplies column (A row) l % 16 and, with j = l / 16, the k's
+// 32 j + 8 q + 0..7 of a block for MFMA q, so a lane's 16 bytes are the weight words of four
+// MFMAs. Loading them that way makes four neighbouring lanes touch four rows (the L1 looks
+// up a line per lane); instead 4 lanes take 64 consecutive bytes of a row, A rows go 256
+// bytes at a time, and both pass through the wave's own LDS space (no barrier), A in the
+// dequant's pair order. A block's loads are issued during the block before it.
+// Bound: VALU issue (the exact dequant, 13 per 8 weights, and the staging) and the L1's
+// lookups (39 and 77 % of the cycles at 8 x 19456 x 2560 before the staging), with the
+// tiles on the busiest CU. Four blocks of loads in flight instead of one were slower (most
+// waves run 3-5 blocks, and the surplus loads cost lookups). M = 8, us against the 128-column
+// tiles of 32 or 128 rows it replaces (60 to 152 workgroups): 2560 x 9728 22.6 -> 9.5,
+// 19456 x 2560 26.7 -> 12.5, 6144 x 2560 10.9 -> 5.3, 4096 x 1024 6.8 -> 3.4; M = 24: 23.1 ->
+// 15.2, 27.5 -> 15.6, 11.8 -> 7.6, 7.1 -> 4.2.
+template <int AR, int NT, int WV>
+__global__ __launch_bounds__(64 * WV) void w4g_skinny_kernel(const __half* __restrict__ a, uint32_t lda,
+                                                             const uint8_t* __restrict__ wq,
+                                                             const __half* __restrict__ ws, __half* __restrict__ y,
+                                                             uint32_t ldy, uint32_t M, uint32_t N, uint32_t K,
+                                                             const __half* __restrict__ res, uint32_t ldr, int swiglu) {
+    typedef float f4_t __attribute__((ext_vector_type(4)));
+    constexpr int MT = (AR + 15) / 16, NA = AR / 4;   // row tiles; A loads per block (4 rows each)
+    constexpr uint32_t AS = 272, WS = 80;             // staged row strides of A and W, bytes
+    constexpr uint32_t WOFF = AR * AS, SOFF = WOFF + NT * 16 * WS;
+    constexpr uint32_t STAGE = SOFF + NT * 128, RED = MT * NT * 1024;   // bytes per wave
+    __shared__ __align__(16) uint8_t lds[WV * (STAGE > RED ? STAGE : RED)];
+    float* red = reinterpret_cast<float*>(lds);
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, j4 = lane >> 4, l16 = lane & 15;
+    const uint32_t r4 = lane >> 2, c4 = lane & 3;     // W as loaded: row r4 of the tile, chunk c4 of the block
+    const uint32_t n0 = blockIdx.x * (16 * NT), G = K / 64, nch = K / 32;   // nch: 32-deep chunks of a row
+    const uint32_t nblk = (nch + 3) / 4, per = (nblk + WV - 1) / WV;
+    const uint32_t b0 = min(wave * per, nblk), b1 = min(b0 + per, nblk);
+    const uint8_t* wt = wq + (size_t)n0 * (K / 2);
+    const uint16_t* st0 = reinterpret_cast<const uint16_t*>(ws) + (size_t)n0 * G;
+    uint32_t nr[NT];   // tile row of each W load, inside [0, N - n0)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) nr[t] = min(16 * t + r4, N - 1 - n0);
+    uint8_t* st = lds + wave * STAGE;
+    const __half* arow[NA];   // rows lane / 16 + 4 i
+#pragma unroll
+    for (int i = 0; i < NA; ++i) arow[i] = a + (size_t)min(4 * i + j4, M - 1) * lda;
+
+    u32x4 rw[NT], ra[NA];
+    uint16_t rs[NT];
+    auto load = [&](uint32_t b) __attribute__((always_inline)) {
+        const uint32_t c = min(4 * b + c4, nch - 1), ca = min(16 * b + l16, 4 * nch - 1);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            rw[t] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wt + (nr[t] * (K / 2) + 16 * c)));
+            rs[t] = st0[nr[t] * G + (c >> 1)];
+        }
+#pragma unroll
+        for (int i = 0; i < NA; ++i) ra[i] = *reinterpret_cast<const u32x4*>(arow[i] + 8 * ca);
+    };
+    f4_t acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[i][t] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+
+    load(min(b0, nblk - 1));
+#pragma unroll 1
+    for (uint32_t b = b0; b < b1; ++b) {
+        if (4 * b + 4 > nch) {   // the half block: chunks past K count as zero weights and activations
+#pragma unroll
+            for (int i = 0; i < NA; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) ra[i][e] = 16 * b + l16 < 4 * nch ? ra[i][e] : 0u;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) rs[t] = 4 * b + c4 < nch ? rs[t] : (uint16_t)0;
+        }
+#pragma unroll
+        for (int i = 0; i < NA; ++i) *reinterpret_cast<u32x4*>(st + (4 * i + j4) * AS + 16 * l16) = pair_order16(ra[i]);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            *reinterpret_cast<u32x4*>(st + WOFF + (16 * t + r4) * WS + 16 * c4) = rw[t];
+            *reinterpret_cast<uint16_t*>(st + SOFF + t * 128 + r4 * 8 + 2 * c4) = rs[t];
+        }
+        load(min(b + 1, nblk - 1));
+        __builtin_amdgcn_sched_barrier(0);
+        // lanes read what other lanes of the wave wrote: its DS operations complete in
+        // order, the fences keep the compiler from moving them across
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        u32x4 w[NT];
+        h2_t s2[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            w[t] = *reinterpret_cast<const u32x4*>(st + WOFF + (16 * t + l16) * WS + 16 * j4);
+            const _Float16 sh = *reinterpret_cast<const _Float16*>(st + SOFF + t * 128 + l16 * 8 + 2 * j4);
+            s2[t] = h2_t{sh, sh};
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            h8_t af[MT];
+#pragma unroll
+            for (int i = 0; i < MT; ++i)   // of AR = 8 rows the tile's second half repeats them (not stored)
+                af[i] = *reinterpret_cast<const h8_t*>(st + ((16 * i + l16) % AR) * AS + 64 * j4 + 16 * q);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                h2_t d[4];
+                dequant_word(w[t][q], s2[t], d);
+                const h8_t bf = {d[0][0], d[0][1], d[1][0], d[1][1], d[2][0], d[2][1], d[3][0], d[3][1]};
+#pragma unroll
+                for (int i = 0; i < MT; ++i) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i], bf, acc[i][t], 0, 0, 0);
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+
+    // Accumulator layout (16x16): lane l, reg r -> col l%16, row 4*(l/16) + r.
+    __syncthreads();   // the sums take the staging space
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) *reinterpret_cast<f4_t*>(&red[((wave * MT + i) * NT + t) * 256 + lane * 4]) = acc[i][t];
+    __syncthreads();
+    for (uint32_t it = wave; it < MT * NT; it += WV) {   // one 16 x 16 tile per wave
+        const uint32_t i = it / NT, t = it % NT, col = n0 + 16 * t + l16;
+        f4_t v = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 0; k < WV; ++k) {
+            const f4_t x = *reinterpret_cast<const f4_t*>(&red[(k * MT * NT + it) * 256 + lane * 4]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = __fadd_rn(v[r], x[r]);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t row = 16 * i + 4 * j4 + r;
+            if (!swiglu) {
+                if (row < M && col < N) w4g_store(y, ldy, res, ldr, row, col, v[r]);
+            } else {   // gate in even columns, up in the lane beside
+                const float up = dev::dpp<dev::kDppQuadSwap1>(v[r]);
+                const float act = h2f(silu_f16_expr(f2hb(v[r])));
+                uint16_t o = f2hb(__fmul_rn(act, h2f(f2hb(up))));
+                if (row < M && col < N && !(l16 & 1)) {
+                    const uint32_t oc = col >> 1;
+                    if (res) o = f2hb(__fadd_rn(h2f(o), h2f(__builtin_bit_cast(uint16_t, res[(size_t)row * ldr + oc]))));
+                    reinterpret_cast<uint16_t*>(y)[(size_t)row * ldy + oc] = o;
+                }
+            }
+        }
+    }
+}
+
 // Wide variant for the wide-N shapes: a 128 x 256 workgroup tile, each wave 128 x 64
 // (4 x 2 MFMA tiles), so every A fragment read from LDS feeds two MFMAs (half the LDS
 // read traffic per MFMA of the 128 x 128 tile, whose A reads keep LDS as busy as the
@@ -1206,6 +1356,30 @@ hipError_t launch_w4g_gemm(const __half* a, uint32_t lda, const uint8_t* wq, con
                            nt, K / GB_K, nullptr, R);
         return hipGetLastError();
     }
+    if (w4g_gemm_skinny(M)) {
+        const uint32_t tiles = (N + 15) / 16, cu = (uint32_t)device_cu_count();
+        auto go = [&](auto kern, uint32_t nt, uint32_t wv) {
+            hipLaunchKernelGGL(kern, dim3((tiles + nt - 1) / nt), dim3(64 * wv), 0, st, a, lda, wq, ws, y, ldy, M, N, K,
+                               epi.res, epi.ldr, epi.swiglu ? 1 : 0);
+            return hipGetLastError();
+        };
+        // Column tiles per workgroup: the fewest on the busiest CU, then the widest (A is
+        // staged once per workgroup). M = 8, us at NT = 1 / 2 / 3 / 5 (8 waves, 4 from NT = 3):
+        // 2560 x 9728 9.5 / 14.1 / 19.8 / 29.6, 6144 x 2560 5.5 / 5.3 / 6.2 / 8.6, 19456 x 2560
+        // 15.5 / 14.2 / 13.1 / 12.5 (1216 tiles: 5 on the busiest CU with 1 or 5, 6 with 2 or 3).
+        uint32_t nt = 1, best = ~0u;
+        for (uint32_t c : {1u, 2u, 3u, 5u}) {
+            const uint32_t busiest = ((tiles + c - 1) / c + cu - 1) / cu * c;
+            if (busiest <= best) { best = busiest; nt = c; }
+        }
+        auto rows = [&](auto ar) {
+            constexpr int AR = decltype(ar)::value;
+            return nt == 1 ? go(w4g_skinny_kernel<AR, 1, 8>, 1, 8) : nt == 2 ? go(w4g_skinny_kernel<AR, 2, 8>, 2, 8)
+                 : nt == 3 ? go(w4g_skinny_kernel<AR, 3, 4>, 3, 4) : go(w4g_skinny_kernel<AR, 5, 4>, 5, 4);
+        };
+        return M <= 8 ? rows(std::integral_constant<int, 8>{}) : M <= 16 ? rows(std::integral_constant<int, 16>{})
+                                                                       : rows(std::integral_constant<int, 32>{});
+    }
     if (epi.swiglu) {
         const hipError_t te = silu_table_ready(st);
         if (te != hipSuccess) return te;
@@ -1280,6 +1454,7 @@ hipError_t launch_w4g_gemm(const __half* a, uint32_t lda, const uint8_t* wq, con
 // M = 128, N = 2560, K = 9728 58.2 -> 24.6 us);
 // otherwise two parts of 16+ steps on the 128 x 128 kernel.
 uint32_t w4g_gemm_split_parts(uint32_t M, uint32_t N, uint32_t K) {
+    if (w4g_gemm_skinny(M)) return 1u;   // that kernel splits K inside its workgroups
     const size_t mt = (M + GB_M - 1) / GB_M, cus = (size_t)device_cu_count();
     if (mt * ((N + GB_N - 1) / GB_N) >= 2 * cus) return 1u;
     if (K / GB_K >= 48 && 3 * mt * ((N + GW_N - 1) / GW_N) <= 2 * cus) return 3u;

@@ -66,6 +66,9 @@ hipError_t launch_w4g_gemm(const __half* a, uint32_t lda, const uint8_t* wq, con
                            hipStream_t st, const W4gEpilogue& epi = W4gEpilogue());
 // K parts the GEMM uses for (M, N, K) when given a workspace, and the workspace bytes
 // (0 when it runs unsplit).
+// M <= 32 rows run w4g_skinny_kernel (K split inside its workgroups) unless the call
+// carries the RoPE epilogue.
+inline bool w4g_gemm_skinny(uint32_t M) { return M <= 32; }
 uint32_t w4g_gemm_split_parts(uint32_t M, uint32_t N, uint32_t K);
 size_t w4g_gemm_split_bytes(uint32_t M, uint32_t N, uint32_t K);
 // w[n*K + k] = fp16(q * s) (bit-exact dequant; used by tests and the fp16 fallback).

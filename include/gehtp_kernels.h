@@ -44,7 +44,8 @@ int gehtp_w4g_fused(const void* x, uint32_t ldx, const void* wq, const void* ws,
                     uint32_t ldy, uint32_t M, uint32_t N, uint32_t K, const void* gamma,
                     const void* res, uint32_t ldr, uint32_t mode, void* stream);
 /* gehtp_w4g_fused with an fp32 workspace (16-byte aligned) that lets the GEMM split K for
- * narrow-N shapes (fewer 128 x 128 tiles than two per CU): in three parts (K >= 48 * 64)
+ * narrow-N shapes of more than 32 rows (fewer 128 x 128 tiles than two per CU; up to 32
+ * rows run a kernel that splits K inside its workgroups): in three parts (K >= 48 * 64)
  * when the 128 x 256 grid of three parts fits one round at two workgroups per CU (on
  * that tile when the grid also reaches half the CUs, else on 128-column tiles of 128,
  * 64 or 32 rows), else in two (K >= 32 * 64) on the 128-column tiles; each part writes

@@ -778,3 +778,50 @@ def test_matmul_f16_tiles_and_edges(lib, torch_dev, M, K, N, Bn):
                                                                                    ref[~ok & ~torch.isnan(ref)]), what
             err = (win - ref)[ok].abs()
             assert (err <= ref[ok].abs() * 2 ** -11 + mag[ok] * K * 2 ** -24 + 2 ** -24).all(), (what, float(err.max()))
+
+
+@pytest.mark.parametrize("M,N,K,mode,use_res,pad", [(5, 16, 64, 0, False, 0), (8, 1, 192, 0, True, 0), (9, 250, 576, 1, False, 8),
+                                                    (16, 4112, 1024, 0, False, 0), (17, 6150, 2560, 1, True, 0),
+                                                    (32, 12320, 128, 0, True, 8), (31, 20482, 448, 1, True, 0),
+                                                    (8, 2560, 9728, 0, True, 0)])
+def test_w4g_gemm_few_rows(lib, oracle, torch_dev, M, N, K, mode, use_res, pad):
+    """M <= 32: 8, 16 or 32 staged rows, 1, 2, 3 or 5 column tiles per workgroup on 256 CUs
+    (N up to 4096 / 8192 / 12288 / beyond), partial row and column tiles, fewer K blocks than
+    waves, a half block at the end (K % 128 = 64), padded x and y rows, both epilogues.
+    Against the oracle: the fp32 sums differ in order only, so an output rounds to the
+    neighbouring fp16 value at most where no further op follows (one ulp, 2^-10 of the value,
+    beside the order's own K 2^-24 of the summed magnitudes); an infinite activation stays in
+    its row."""
+    import torch
+    rng = np.random.default_rng(M + N + K)
+    n_out = N // 2 if mode else N
+    _, wq, ws = w4g_weights(rng, N, K)
+    x = normal_f16(rng, M, K + pad) * np.float16(0.25)
+    res = normal_f16(rng, M, n_out)
+    xd, wd, sd, rd = (to_dev(v, torch_dev) for v in (x, wq, ws, res))
+
+    def run():
+        y = torch.full((M, n_out + pad), 7.0, dtype=torch.float16, device=torch_dev)
+        assert lib.gehtp_w4g_split_bytes(M, N, K) == 0
+        assert lib.gehtp_w4g_fused(ptr(xd), K + pad, ptr(wd), ptr(sd), ptr(y), n_out + pad, M, N, K, None,
+                                   ptr(rd) if use_res else None, n_out, mode, stream_ptr()) == 0
+        _sync()
+        got = from_dev(y)
+        assert (got[:, n_out:] == 7).all()
+        return got[:, :n_out]
+
+    got = run()
+    xc = np.ascontiguousarray(x[:, :K])
+    acc = oracle.matmul_w4g(xc, wq, ws, threads=8)
+    ref = oracle.binary(oracle.unary(acc[:, 0::2].copy(), 12), acc[:, 1::2].copy(), 2) if mode else acc
+    if use_res:
+        ref = oracle.binary(ref, res, 0)
+    assert_close(got, ref, what=f"{M}x{N}x{K} mode={mode} res={use_res}")
+    if not mode and not use_res:
+        mag = np.abs(xc).astype(np.float64) @ np.abs(oracle.w4g_dequant(wq, ws, K).astype(np.float64)).T
+        err = np.abs(got.astype(np.float64) - ref.astype(np.float64))
+        assert (err <= np.abs(ref.astype(np.float64)) * 2.0 ** -10 + mag * K * 2.0 ** -24 + 2.0 ** -24).all()
+    xd[M - 1, K - 1] = float("inf")
+    hot = run()
+    assert np.array_equal(hot[:M - 1].view(np.uint16), got[:M - 1].view(np.uint16))
+    assert not np.isfinite(hot[M - 1].astype(np.float32)).all()
