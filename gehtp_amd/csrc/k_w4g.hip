@@ -704,7 +704,7 @@ __global__ __launch_bounds__(256, 3) void w4g_gemm_kernel(
 
 // ---------------------------------------------------------------------------
 // GEMM of few rows (M <= 32): weights stream once, so a tile is 16 NT columns of all M rows
-// (AR >= M of them staged) and K is split over the workgroup's WV waves in contiguous ranges
+// (AR >= M of them staged; with NORM, M <= 4, normalized as they are staged) and K is split over the workgroup's WV waves in contiguous ranges
 // of 128-deep blocks, their sums added in LDS in wave order; no workspace, one launch. On
 // v_mfma_f32_16x16x32_f16 lane l supplies column (A row) l % 16 and, with j = l / 16, the k's
 // 32 j + 8 q + 0..7 of a block for MFMA q, so a lane's 16 bytes are the weight words of four
@@ -719,12 +719,14 @@ __global__ __launch_bounds__(256, 3) void w4g_gemm_kernel(
 // tiles of 32 or 128 rows it replaces (60 to 152 workgroups): 2560 x 9728 22.6 -> 9.5,
 // 19456 x 2560 26.7 -> 12.5, 6144 x 2560 10.9 -> 5.3, 4096 x 1024 6.8 -> 3.4; M = 24: 23.1 ->
 // 15.2, 27.5 -> 15.6, 11.8 -> 7.6, 7.1 -> 4.2.
-template <int AR, int NT, int WV>
+template <int AR, int NT, int WV, bool NORM>
 __global__ __launch_bounds__(64 * WV) void w4g_skinny_kernel(const __half* __restrict__ a, uint32_t lda,
                                                              const uint8_t* __restrict__ wq,
                                                              const __half* __restrict__ ws, __half* __restrict__ y,
                                                              uint32_t ldy, uint32_t M, uint32_t N, uint32_t K,
-                                                             const __half* __restrict__ res, uint32_t ldr, int swiglu) {
+                                                             const __half* __restrict__ res, uint32_t ldr, int swiglu,
+                                                             const __half* __restrict__ gamma) {
+    static_assert(!NORM || AR == 4, "one row per 16 lanes");
     typedef float f4_t __attribute__((ext_vector_type(4)));
     constexpr int MT = (AR + 15) / 16, NA = AR / 4;   // row tiles; A loads per block (4 rows each)
     constexpr uint32_t AS = 272, WS = 80;             // staged row strides of A and W, bytes
@@ -747,7 +749,7 @@ __global__ __launch_bounds__(64 * WV) void w4g_skinny_kernel(const __half* __res
 #pragma unroll
     for (int i = 0; i < NA; ++i) arow[i] = a + (size_t)min(4 * i + j4, M - 1) * lda;
 
-    u32x4 rw[NT], ra[NA];
+    u32x4 rw[NT], ra[NA], rg;
     uint16_t rs[NT];
     auto load = [&](uint32_t b) __attribute__((always_inline)) {
         const uint32_t c = min(4 * b + c4, nch - 1), ca = min(16 * b + l16, 4 * nch - 1);
@@ -758,6 +760,7 @@ __global__ __launch_bounds__(64 * WV) void w4g_skinny_kernel(const __half* __res
         }
 #pragma unroll
         for (int i = 0; i < NA; ++i) ra[i] = *reinterpret_cast<const u32x4*>(arow[i] + 8 * ca);
+        if constexpr (NORM) rg = *reinterpret_cast<const u32x4*>(gamma + 8 * ca);
     };
     f4_t acc[MT][NT];
 #pragma unroll
@@ -766,8 +769,54 @@ __global__ __launch_bounds__(64 * WV) void w4g_skinny_kernel(const __half* __res
         for (int t = 0; t < NT; ++t) acc[i][t] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
     load(min(b0, nblk - 1));
+    float rms = 1.0f, rcp = 1.0f;   // of this lane's A row
+    if constexpr (NORM) {   // RMSNorm of the rows as in w4g_gemv_kernel: squares in double, the whole row
+        __shared__ double s_ss[WV][AR];
+        double ss[AR];
+#pragma unroll
+        for (int m = 0; m < AR; ++m) ss[m] = 0.0;
+        for (uint32_t i = tid; i < K / 8; i += 64 * WV) {   // every row's loads first
+            u32x4 v[AR];
+#pragma unroll
+            for (int m = 0; m < AR; ++m)
+                v[m] = reinterpret_cast<const u32x4*>(a + (size_t)min((uint32_t)m, M - 1) * lda)[i];
+#pragma unroll
+            for (int m = 0; m < AR; ++m)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const double lo = (double)h2f((uint16_t)(v[m][e] & 0xFFFFu)), hi = (double)h2f((uint16_t)(v[m][e] >> 16));
+                    ss[m] = __builtin_fma(lo, lo, ss[m]);
+                    ss[m] = __builtin_fma(hi, hi, ss[m]);
+                }
+        }
+#pragma unroll
+        for (int m = 0; m < AR; ++m) {
+            const double w = dev::wave_sum(ss[m]);
+            if (lane == 0) s_ss[wave][m] = w;
+        }
+        __syncthreads();
+        double tot = 0.0;
+#pragma unroll
+        for (int v = 0; v < WV; ++v) tot += s_ss[v][j4];
+        rms = (float)sqrt(tot / (double)K + 1e-6);
+        rcp = __fdiv_rn(1.0f, rms);
+    }
 #pragma unroll 1
     for (uint32_t b = b0; b < b1; ++b) {
+        if constexpr (NORM) {   // x / rms (Markstein) * gamma + 0, rounded to fp16
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float v[2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const float x = h2f((uint16_t)(ra[0][e] >> (16 * h))), q = x * rcp;
+                    const float d = __builtin_fmaf(__builtin_fmaf(-q, rms, x), rcp, q);
+                    v[h] = __builtin_fmaf(d, h2f((uint16_t)(rg[e] >> (16 * h))), 0.0f);
+                }
+                asm volatile("" : "+v"(v[0]), "+v"(v[1]));   // the f32 result, rounded before the conversion
+                ra[0][e] = (uint32_t)f2hb(v[0]) | ((uint32_t)f2hb(v[1]) << 16);
+            }
+        }
         if (4 * b + 4 > nch) {   // the half block: chunks past K count as zero weights and activations
 #pragma unroll
             for (int i = 0; i < NA; ++i)
@@ -801,7 +850,7 @@ __global__ __launch_bounds__(64 * WV) void w4g_skinny_kernel(const __half* __res
         for (int q = 0; q < 4; ++q) {
             h8_t af[MT];
 #pragma unroll
-            for (int i = 0; i < MT; ++i)   // of AR = 8 rows the tile's second half repeats them (not stored)
+            for (int i = 0; i < MT; ++i)   // of AR = 4 or 8 rows the rest of the tile repeats them (not stored)
                 af[i] = *reinterpret_cast<const h8_t*>(st + ((16 * i + l16) % AR) * AS + 64 * j4 + 16 * q);
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
@@ -1267,6 +1316,37 @@ bool gemv_rw_launch(const GemvRwArgs& A, hipStream_t st, hipError_t* err) {
     return true;
 }
 
+// Launch of w4g_skinny_kernel for M <= 32 rows (with epi.gamma: M <= 4).
+static hipError_t launch_skinny(const __half* a, uint32_t lda, const uint8_t* wq, const __half* ws, __half* y, uint32_t ldy,
+                                uint32_t M, uint32_t N, uint32_t K, hipStream_t st, const W4gEpilogue& epi) {
+    const uint32_t tiles = (N + 15) / 16, cu = (uint32_t)device_cu_count();
+    auto go = [&](auto kern, uint32_t nt, uint32_t wv) {
+        hipLaunchKernelGGL(kern, dim3((tiles + nt - 1) / nt), dim3(64 * wv), 0, st, a, lda, wq, ws, y, ldy, M, N, K,
+                           epi.res, epi.ldr, epi.swiglu ? 1 : 0, epi.gamma);
+        return hipGetLastError();
+    };
+    // Column tiles per workgroup: the fewest on the busiest CU, then the widest (A is
+    // staged once per workgroup). M = 8, us at NT = 1 / 2 / 3 / 5 (8 waves, 4 from NT = 3):
+    // 2560 x 9728 9.5 / 14.1 / 19.8 / 29.6, 6144 x 2560 5.5 / 5.3 / 6.2 / 8.6, 19456 x 2560
+    // 15.5 / 14.2 / 13.1 / 12.5 (1216 tiles: 5 on the busiest CU with 1 or 5, 6 with 2 or 3).
+    uint32_t nt = 1, best = ~0u;
+    for (uint32_t c : {1u, 2u, 3u, 5u}) {
+        const uint32_t busiest = ((tiles + c - 1) / c + cu - 1) / cu * c;
+        if (busiest <= best) { best = busiest; nt = c; }
+    }
+    auto rows = [&](auto ar, auto norm) {
+        constexpr int AR = decltype(ar)::value;
+        constexpr bool NO = decltype(norm)::value;
+        return nt == 1 ? go(w4g_skinny_kernel<AR, 1, 8, NO>, 1, 8) : nt == 2 ? go(w4g_skinny_kernel<AR, 2, 8, NO>, 2, 8)
+             : nt == 3 ? go(w4g_skinny_kernel<AR, 3, 4, NO>, 3, 4) : go(w4g_skinny_kernel<AR, 5, 4, NO>, 5, 4);
+    };
+    if (epi.gamma) return rows(std::integral_constant<int, 4>{}, std::true_type{});
+    return M <= 4    ? rows(std::integral_constant<int, 4>{}, std::false_type{})
+         : M <= 8  ? rows(std::integral_constant<int, 8>{}, std::false_type{})
+         : M <= 16 ? rows(std::integral_constant<int, 16>{}, std::false_type{})
+                   : rows(std::integral_constant<int, 32>{}, std::false_type{});
+}
+
 hipError_t launch_w4g_gemv(const __half* x, uint32_t ldx, const uint8_t* wq, const __half* ws,
                            __half* y, uint32_t ldy, uint32_t M, uint32_t N, uint32_t K,
                            hipStream_t st, const W4gEpilogue& epi) {
@@ -1283,6 +1363,13 @@ hipError_t launch_w4g_gemv(const __half* x, uint32_t ldx, const uint8_t* wq, con
         hipError_t e = hipSuccess;
         if (gemv_rw_launch(GemvRwArgs{x, wq, ws, y, N, K, epi.gamma, epi.res, epi.swiglu ? 1 : 0}, st, &e)) return e;
     }
+    // Three or four rows, and two with the RMSNorm (whose prologue this kernel repeats in
+    // every workgroup, for all rows at once), run faster as a GEMM: us, this kernel against
+    // w4g_skinny_kernel, M = 2 / 3 / 4: 19456 x 2560 with the RMSNorm 18.2 / 28.6 / 42.9
+    // against 13.3 / 13.4 / 13.4, without 10.5 / 15.3 / 16.8 against 11.4 / 11.5 / 11.5;
+    // 4096 x 1024 8.2 / 10.5 / 12.3 against 4.3 / 4.3 / 4.4, 3.7 / 4.3 / 4.8 against
+    // 3.2 / 3.1 / 3.2 (2560 x 9728, M = 2, without: 7.4 against 9.2).
+    if (M >= 3 || (M == 2 && epi.gamma)) return launch_skinny(x, ldx, wq, ws, y, ldy, M, N, K, st, epi);
     // Rows per workgroup: about two workgroups per CU (three when one workgroup holds a
     // single row per pass, as for K = 9728: measured 11 % faster there, slower for the
     // multi-row shapes), partial sums within 32 KiB.
@@ -1317,8 +1404,6 @@ hipError_t launch_w4g_gemv(const __half* x, uint32_t ldx, const uint8_t* wq, con
     switch (M) {
     case 1: return gemv_dispatch<1>(g3, b3, lds, st, A);
     case 2: return gemv_dispatch<2>(g3, b3, lds, st, A);
-    case 3: return gemv_dispatch<3>(g3, b3, lds, st, A);
-    case 4: return gemv_dispatch<4>(g3, b3, lds, st, A);
     default: return hipErrorInvalidValue;
     }
 }
@@ -1356,30 +1441,7 @@ hipError_t launch_w4g_gemm(const __half* a, uint32_t lda, const uint8_t* wq, con
                            nt, K / GB_K, nullptr, R);
         return hipGetLastError();
     }
-    if (w4g_gemm_skinny(M)) {
-        const uint32_t tiles = (N + 15) / 16, cu = (uint32_t)device_cu_count();
-        auto go = [&](auto kern, uint32_t nt, uint32_t wv) {
-            hipLaunchKernelGGL(kern, dim3((tiles + nt - 1) / nt), dim3(64 * wv), 0, st, a, lda, wq, ws, y, ldy, M, N, K,
-                               epi.res, epi.ldr, epi.swiglu ? 1 : 0);
-            return hipGetLastError();
-        };
-        // Column tiles per workgroup: the fewest on the busiest CU, then the widest (A is
-        // staged once per workgroup). M = 8, us at NT = 1 / 2 / 3 / 5 (8 waves, 4 from NT = 3):
-        // 2560 x 9728 9.5 / 14.1 / 19.8 / 29.6, 6144 x 2560 5.5 / 5.3 / 6.2 / 8.6, 19456 x 2560
-        // 15.5 / 14.2 / 13.1 / 12.5 (1216 tiles: 5 on the busiest CU with 1 or 5, 6 with 2 or 3).
-        uint32_t nt = 1, best = ~0u;
-        for (uint32_t c : {1u, 2u, 3u, 5u}) {
-            const uint32_t busiest = ((tiles + c - 1) / c + cu - 1) / cu * c;
-            if (busiest <= best) { best = busiest; nt = c; }
-        }
-        auto rows = [&](auto ar) {
-            constexpr int AR = decltype(ar)::value;
-            return nt == 1 ? go(w4g_skinny_kernel<AR, 1, 8>, 1, 8) : nt == 2 ? go(w4g_skinny_kernel<AR, 2, 8>, 2, 8)
-                 : nt == 3 ? go(w4g_skinny_kernel<AR, 3, 4>, 3, 4) : go(w4g_skinny_kernel<AR, 5, 4>, 5, 4);
-        };
-        return M <= 8 ? rows(std::integral_constant<int, 8>{}) : M <= 16 ? rows(std::integral_constant<int, 16>{})
-                                                                       : rows(std::integral_constant<int, 32>{});
-    }
+    if (w4g_gemm_skinny(M)) return launch_skinny(a, lda, wq, ws, y, ldy, M, N, K, st, epi);
     if (epi.swiglu) {
         const hipError_t te = silu_table_ready(st);
         if (te != hipSuccess) return te;

@@ -32,7 +32,8 @@ extern "C" {
  * K % 64 == 0, ldx % 8 == 0, x and wq 16-byte aligned. */
 int gehtp_w4g_matmul(const void* x, uint32_t ldx, const void* wq, const void* ws, void* y,
                      uint32_t ldy, uint32_t M, uint32_t N, uint32_t K, void* stream);
-/* Force one implementation (for measurement): GEMV needs M <= 4. */
+/* Force one side of that choice (for measurement): GEMV needs M <= 4 (3 and 4 rows run the
+ * GEMM of few rows either way). */
 int gehtp_w4g_gemv(const void* x, uint32_t ldx, const void* wq, const void* ws, void* y,
                    uint32_t ldy, uint32_t M, uint32_t N, uint32_t K, void* stream);
 int gehtp_w4g_gemm(const void* x, uint32_t ldx, const void* wq, const void* ws, void* y,

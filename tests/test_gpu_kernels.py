@@ -825,3 +825,28 @@ def test_w4g_gemm_few_rows(lib, oracle, torch_dev, M, N, K, mode, use_res, pad):
     hot = run()
     assert np.array_equal(hot[:M - 1].view(np.uint16), got[:M - 1].view(np.uint16))
     assert not np.isfinite(hot[M - 1].astype(np.float32)).all()
+
+
+@pytest.mark.parametrize("M,N,K,mode,use_res", [(2, 40, 64, 0, True), (2, 6150, 2560, 1, True), (3, 4096, 192, 0, False),
+                                                (3, 12290, 1024, 0, False), (4, 19456, 2560, 1, False), (4, 33, 8192, 0, True)])
+def test_w4g_few_rows_norm(lib, oracle, torch_dev, M, N, K, mode, use_res):
+    """2 to 4 rows with the RMSNorm inside the call: the 16-column tiles normalize the rows
+    as they stage them (1, 2, 3 or 5 tiles per workgroup, K blocks fewer than waves, a half
+    block at the end, the longest K the call takes). Against the oracle's RMSNorm, linear
+    and epilogue."""
+    import torch
+    rng = np.random.default_rng(7 * M + N + K)
+    n_out = N // 2 if mode else N
+    _, wq, ws = w4g_weights(rng, N, K)
+    x, gamma = normal_f16(rng, M, K), (rng.uniform(0.8, 1.2, K) * 0.25).astype(np.float16)
+    res = normal_f16(rng, M, n_out)
+    y = torch.empty((M, n_out), dtype=torch.float16, device=torch_dev)
+    assert lib.gehtp_w4g_fused(ptr(to_dev(x, torch_dev)), K, ptr(to_dev(wq, torch_dev)), ptr(to_dev(ws, torch_dev)),
+                               ptr(y), n_out, M, N, K, ptr(to_dev(gamma, torch_dev)),
+                               ptr(to_dev(res, torch_dev)) if use_res else None, n_out, mode, stream_ptr()) == 0
+    _sync()
+    acc = oracle.matmul_w4g(oracle.rmsnorm2(x, gamma, np.zeros(K, np.float16)), wq, ws, threads=8)
+    ref = oracle.binary(oracle.unary(acc[:, 0::2].copy(), 12), acc[:, 1::2].copy(), 2) if mode else acc
+    if use_res:
+        ref = oracle.binary(ref, res, 0)
+    assert_close(from_dev(y), ref, what=f"norm {M}x{N}x{K} mode={mode} res={use_res}")
