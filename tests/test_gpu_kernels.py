@@ -850,3 +850,28 @@ def test_w4g_few_rows_norm(lib, oracle, torch_dev, M, N, K, mode, use_res):
     if use_res:
         ref = oracle.binary(ref, res, 0)
     assert_close(from_dev(y), ref, what=f"norm {M}x{N}x{K} mode={mode} res={use_res}")
+
+
+@pytest.mark.parametrize("rows,n", [(1, 1), (9, 2), (5, 63), (3, 64), (70, 32), (6, 129), (3, 255), (2, 257), (7, 511), (1030, 512), (4, 513), (9, 1024), (1100, 1001),
+                                    (6, 2048), (5, 2049), (5, 7)])
+def test_softmax_row_per_wave(lib, torch_dev, rows, n):
+    """The row-per-wave softmax (n <= 2048: chunks of 1, 2, 4 or 8 values, 1, 2 or 4 per lane, one
+    or four rows per workgroup) and the longer rows beside it, at row lengths off every alignment, from a
+    pointer 2 bytes off, in place, with -inf entries (a masked row's shape). Against float64:
+    one fp16 rounding of the exponential and one of the quotient (2^-10 together), the fp32
+    exponential and sum (n 2^-24) besides."""
+    import torch
+    g = torch.Generator(device=torch_dev).manual_seed(rows * 3 + n)
+    x = (torch.randn((rows, n), device=torch_dev, generator=g) * 3).half()
+    x[rows // 2, n // 2 + 1:] = float("-inf")
+    for off in (0, 1):
+        buf = torch.full((rows * n + off + 8,), 7.0, dtype=torch.float16, device=torch_dev)
+        buf[off:off + rows * n] = x.reshape(-1)
+        p = buf.data_ptr() + 2 * off
+        assert lib.gehtp_softmax(p, p, rows, n, stream_ptr()) == 0
+        _sync()
+        assert (buf[:off] == 7).all() and (buf[off + rows * n:] == 7).all()
+        got = buf[off:off + rows * n].view(rows, n).double()
+        ref = torch.softmax(x.double(), -1)
+        err = (got - ref).abs()
+        assert (err <= ref * (2 ** -10 + (n + 16) * 2 ** -24) + 2 ** -24).all(), (off, float(err.max()))
