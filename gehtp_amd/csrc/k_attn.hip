@@ -46,8 +46,7 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const _Float16* p) {
 }
 
 // Flash attention forward. A workgroup owns 32 WPH queries of one head (wave w of a
-// half: queries 32w..32w+31; WPH = 4 normally, 2 when 128-query tiles would leave CUs
-// idle, 1 when 64-query tiles would too); per 64-key stage, K and V are staged row-major in LDS (the next stage's
+// part: queries 32w..32w+31); per 64-key stage, K and V are staged row-major in LDS (the next stage's
 // loads are in flight during the compute). Scores are computed transposed,
 // S^T = K Q^T (MFMA A = K rows, B = Q^T held in registers), so each lane owns one query
 // and its 32 scores of a stage; the online-softmax statistics need one exchange with
@@ -57,28 +56,33 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const _Float16* p) {
 // The online softmax keeps a lazily moved reference max (see the stage code) and sums
 // the fp16 weights P.V consumes; K / V stage rows come in through buffer loads.
 //
-// Two halves of WPH waves split a tile's key stages: half p runs stages
-// [p*ns0, min(ns, (p+1)*ns0)) (ns0 = ceil(ns/2)) on its own LDS tiles, both halves in
-// lockstep (the shorter one idles through its last step), and half 1 hands its partial
-// (O, max, sum) to half 0 through LDS at the end. A causal tile then costs half its
-// stages: the heaviest tiles no longer set the kernel's time (the grid runs the heavy
-// tiles of every head first, one 8-wave workgroup per CU, the light ones behind them).
-constexpr uint32_t KV_HALF = KT * KS + KT * VSR;   // halves of one LDS K + V stage
+// NP parts of WPH waves split a tile's key stages: part p runs stages
+// [p*ns0, min(ns, (p+1)*ns0)) (ns0 = ceil(ns/NP)) on its own LDS tiles, all parts in
+// lockstep (a shorter one idles through its last step), and the partial (O, max, sum)s
+// meet through LDS at the end. A causal tile then costs 1/NP of its stages: the heaviest
+// tiles no longer set the kernel's time (the grid runs the heavy tiles of every head
+// first, the light ones behind them).
+//
+// What bounds it: a lone wave per SIMD takes ~1.9 us per stage (32 MFMAs, then ~220
+// vector instructions, little of either overlapped), on top of 4-6 us of launch, first
+// loads and merge. Two parts (2 or 4 waves: one per SIMD at most) double-buffer the
+// stages, 152 KB of LDS, one barrier per stage; four parts give a SIMD two waves at 64
+// queries (3.0 us for their two stages) and half the steps, in the same LDS, one buffer.
+// attn_prefill_form has the rule between the five forms and what each measured.
+constexpr uint32_t KV_HALF = KT * KS + KT * VSR;   // fp16 values of one LDS K + V stage
 
-template <bool CAUSAL, int WPH>
-__global__ __launch_bounds__(128 * WPH) void attn_prefill_kernel(
+template <bool CAUSAL, int WPH, int NP>
+__global__ __launch_bounds__(64 * NP * WPH) void attn_prefill_kernel(
     const __half* __restrict__ q, uint32_t ldq, uint32_t qhs, const __half* __restrict__ k,
     const __half* __restrict__ v, uint32_t ldkv, uint32_t kvhs, __half* __restrict__ out, uint32_t ldo,
     uint32_t ohs, uint32_t S, uint32_t H, uint32_t KVH, float scale_log2) {
-    // 8-wave tiles double-buffer the stages (one workgroup per CU either way); smaller
-    // workgroups keep one buffer, so that two of them still fit a CU's LDS.
-    constexpr bool DB = WPH == 4;
-    __shared__ __align__(16) _Float16 kvbuf[(DB ? 2 : 1) * 2 * KV_HALF];   // [stage buffer][half]
-    constexpr uint32_t QT = 32 * WPH, NT = 64 * WPH;   // queries per tile, threads per half
+    constexpr bool DB = NP == 2;   // two LDS stage buffers
+    __shared__ __align__(16) _Float16 kvbuf[(DB ? 2 : 1) * NP * KV_HALF];   // [stage buffer][part]
+    constexpr uint32_t QT = 32 * WPH, NT = 64 * WPH;   // queries per tile, threads per part
     constexpr int KR = KT * 16 / NT;                     // K / V rows per thread per stage
     const uint32_t part = __builtin_amdgcn_readfirstlane(threadIdx.x / NT), tid = threadIdx.x % NT, lane = tid & 63,
                    wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    _Float16* const Ks0 = kvbuf + part * KV_HALF;   // stage buffer b at + 2 * b * KV_HALF
+    _Float16* const Ks0 = kvbuf + part * KV_HALF;   // stage buffer b at + NP * b * KV_HALF
     const uint32_t n_qt = (S + QT - 1) / QT;
     const uint32_t qtile = n_qt - 1 - blockIdx.y;      // heaviest causal tiles first
     const uint32_t h = blockIdx.x;
@@ -136,15 +140,15 @@ __global__ __launch_bounds__(128 * WPH) void attn_prefill_kernel(
     const uint32_t tr_row = 4 * hl + ((lane & 15) >> 2);
     const uint32_t tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
 
-    const uint32_t ns = (kend + KT - 1) / KT, ns0 = (ns + 1) / 2;
-    const uint32_t st0 = part * ns0, st1 = min(ns, st0 + ns0);   // this half's stages
+    const uint32_t ns = (kend + KT - 1) / KT, ns0 = (ns + NP - 1) / NP;
+    const uint32_t st0 = part * ns0, st1 = min(ns, st0 + ns0);   // this part's stages
     const uint32_t klast = st1 > st0 ? min(st1 * KT, kend) - 1 : kend - 1;
     // With two LDS stage buffers, stage it is computed from buffer it % 2 while the
     // registers hold stage it + 1, written to the other buffer after the compute: one
     // barrier per stage (the other buffer was last read in stage it - 1, before the
     // previous barrier). With one buffer, a barrier before the write as well.
     auto stage_kv = [&](uint32_t b) __attribute__((always_inline)) {
-        _Float16* const Kd = Ks0 + 2 * b * KV_HALF;
+        _Float16* const Kd = Ks0 + NP * b * KV_HALF;
         _Float16* const Vd = Kd + KT * KS;
 #pragma unroll
         for (int i = 0; i < KR; ++i) {
@@ -294,7 +298,7 @@ __global__ __launch_bounds__(128 * WPH) void attn_prefill_kernel(
             }
         }
     };
-    // A stage runs unless it is the shorter half's idle step or wholly masked for this wave.
+    // A stage runs unless it is a shorter part's idle step or wholly masked for this wave.
     auto active = [&](uint32_t it, uint32_t kb) { return st0 + it < st1 && !(CAUSAL && kb > qw + 31); };
     if constexpr (DB) {
         stage_kv(0);
@@ -302,7 +306,7 @@ __global__ __launch_bounds__(128 * WPH) void attn_prefill_kernel(
         __syncthreads();
         for (uint32_t it = 0; it < ns0; ++it) {
             const uint32_t kb = (st0 + it) * KT;
-            const _Float16* const Ks = Ks0 + 2 * (it & 1) * KV_HALF;
+            const _Float16* const Ks = Ks0 + NP * (it & 1) * KV_HALF;
             if (active(it, kb)) stage_compute(Ks, Ks + KT * KS, kb);
             if (it + 1 < ns0) {
                 stage_kv((it + 1) & 1);
@@ -321,8 +325,49 @@ __global__ __launch_bounds__(128 * WPH) void attn_prefill_kernel(
         }
     }
 
-    // Half 1 hands (O, max, sum) to half 0 through the K/V tiles (lane-major floats: 66
-    // per lane, 64 lanes x WPH waves); half 0 rescales both to the common max.
+    if constexpr (NP > 2) {
+        static_assert(NP * 32 == HD && NP * 66 * NT * 4 <= sizeof(kvbuf), "a 32-dim block per part");
+        // Every part leaves its (O, max, sum) in the tiles (lane-major floats, 66 per lane);
+        // part p merges the 32-dim block p of the tile's queries from all of them.
+        __syncthreads();
+        float* const xch = reinterpret_cast<float*>(kvbuf);
+        const uint32_t xl = wave * 64 + lane;
+#pragma unroll
+        for (int dt = 0; dt < HD / 32; ++dt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) xch[(part * 66 + dt * 16 + r) * NT + xl] = o[dt][r];
+        xch[(part * 66 + 64) * NT + xl] = m_run;
+        xch[(part * 66 + 65) * NT + xl] = l_run;
+        __syncthreads();
+        float m = -INFINITY, l = 0.0f, al[NP], acc[16];
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            al[p] = xch[(p * 66 + 64) * NT + xl];
+            m = fmaxf(m, al[p]);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            al[p] = al[p] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((al[p] - m) * scale_log2);
+            l += xch[(p * 66 + 65) * NT + xl] * al[p];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[r] += xch[(p * 66 + part * 16 + r) * NT + xl] * al[p];
+        }
+        if (my_q < S) {
+            const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+            __half* orow = out + (size_t)my_q * ldo + (size_t)h * ohs + part * 32;
+#pragma unroll
+            for (int rb = 0; rb < 4; ++rb) {
+                h4_t v4;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v4[e] = (_Float16)(acc[rb * 4 + e] * inv);
+                *reinterpret_cast<h4_t*>(orow + rb * 8 + 4 * hl) = v4;
+            }
+        }
+    } else {
+    // Part 1 hands (O, max, sum) to part 0 through the K/V tiles (lane-major floats: 66
+    // per lane, 64 lanes x WPH waves); part 0 rescales both to the common max.
     __syncthreads();
     float* xch = reinterpret_cast<float*>(kvbuf);
     const uint32_t xl = wave * 64 + lane;
@@ -359,6 +404,7 @@ __global__ __launch_bounds__(128 * WPH) void attn_prefill_kernel(
                 for (int e = 0; e < 4; ++e) v4[e] = (_Float16)(o[dt][rb * 4 + e] * inv);
                 *reinterpret_cast<h4_t*>(orow + dt * 32 + rb * 8 + 4 * hl) = v4;
             }
+    }
     }
 }
 
@@ -969,6 +1015,50 @@ __global__ __launch_bounds__(256) void merge_oproj_kernel(MergeOprojArgs M) {
                                           M.ws + kWsErr);
 }
 
+// The tile of a prefill: queries per tile (32 wph), parts over the keys, and its measured
+// cost in units of 0.1 us: `base` for a workgroup plus `step` per key stage of a part (one
+// workgroup per CU; S 128..2048, 8/16/32 heads, both masks, fitted within ~5 %).
+//
+// One round of workgroups takes its heaviest member's time. More workgroups than CUs:
+// without a mask all are alike and every begun round costs one; with it, heavy first,
+// the mean load times 1.1 (the tail) once that is larger. Measured, us (32-query x 2
+// parts / 64 x 2 / 128 x 2 / 32 x 4 / 64 x 4), the rule's choice marked:
+//   S  256 x 16 heads causal   *8.2 / 8.9 / 10.6 / 8.2 / 9.7
+//   S  512 x 32 heads causal   18.3 / *13.4 / 15.0 / 19.2 / 13.4
+//   S  768 x 32 heads          44.8 / 30.3 / *18.9 / 38.5 / 30.5
+//   S 1024 x  8 heads causal   19.7 / 19.4 / 21.0 / *16.3 / 17.8
+//   S 1024 x 16 heads causal   25.9 / 20.1 / 22.0 / 24.2 / *18.6
+//   S 1536 x 16 heads          78.3 / 50.4 / *29.6 / 62.3 / 46.4
+//   S 2048 x 32 heads causal   158 / 77 / *52.8 / 134 / 80
+// (The largest tile that still fills the CUs, which stood here before, took 31.8 us for
+// the third line, 52.8 for the sixth: two rounds of 64-query tiles.)
+//
+// Four parts only past 8 stages (S > 512): below, the outputs are the same bits whatever
+// the tile (two parts split the stages of an enclosing tile where it does), and four
+// parts gain nothing up to S = 384 and ~1 us at 512.
+struct AttnTile {
+    uint32_t wph, np, base, step;
+};
+constexpr AttnTile kAttnTiles[5] = {{4, 2, 59, 19}, {2, 2, 47, 18}, {1, 2, 38, 20}, {2, 4, 60, 30}, {1, 4, 49, 28}};
+
+AttnTile attn_prefill_form(uint32_t S, uint32_t H, bool causal) {
+    const uint64_t cus = (uint64_t)device_cu_count(), ns = ((uint64_t)S + KT - 1) / KT;
+    AttnTile best = kAttnTiles[0];
+    uint64_t best_cost = UINT64_MAX;
+    for (const AttnTile& f : kAttnTiles) {
+        if (f.np == 4 && ns <= 8) continue;
+        const uint64_t qt = 32 * f.wph, wgs = (uint64_t)H * ((S + qt - 1) / qt), steps = (ns + f.np - 1) / f.np;
+        uint64_t cost = f.base + f.step * steps;
+        if (!causal) cost *= (wgs + cus - 1) / cus;
+        else if (wgs > cus) cost = std::max(cost, (2 * f.base + f.step * (steps + 1)) * wgs * 11 / (20 * cus));
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = f;
+        }
+    }
+    return best;
+}
+
 }  // namespace
 
 hipError_t launch_attn_prefill(const __half* q, uint32_t ldq, const __half* k, const __half* v,
@@ -985,21 +1075,23 @@ hipError_t launch_attn_prefill_hs(const __half* q, uint32_t ldq, uint32_t qhs, c
     if (!(scale > 0.0f && scale < INFINITY)) return hipErrorInvalidValue;   // the kernel's max needs scale > 0
     if ((uint64_t)ldkv * 2u * KT > 0xFFFFFFFFull) return hipErrorInvalidValue;   // a stage's K / V bytes: 32-bit offsets
     if (!S || !H) return hipSuccess;
-    // 128-query tiles (8-wave workgroups) while they give every CU one; else 64-query
-    // tiles (4-wave workgroups) while those do; else 32-query tiles (2-wave workgroups).
-    const size_t cus = (size_t)device_cu_count();
-    const uint32_t wph = (size_t)H * ((S + 127) / 128) >= cus ? 4u : (size_t)H * ((S + 63) / 64) >= cus ? 2u : 1u;
-    const uint32_t qt = 32 * wph;
-    dim3 grid(H, (S + qt - 1) / qt);   // heads fastest: the heavy tiles of every head go first
+    const AttnTile form = attn_prefill_form(S, H, causal);
     const float sl2 = scale * kLog2e;
-    const auto kern = causal ? (wph == 4   ? attn_prefill_kernel<true, 4>
-                                : wph == 2 ? attn_prefill_kernel<true, 2>
-                                           : attn_prefill_kernel<true, 1>)
-                             : (wph == 4   ? attn_prefill_kernel<false, 4>
-                                : wph == 2 ? attn_prefill_kernel<false, 2>
-                                           : attn_prefill_kernel<false, 1>);
-    hipLaunchKernelGGL(kern, grid, dim3(4 * qt), 0, st, q, ldq, qhs, k, v, ldkv, kvhs, out, ldo, ohs, S, H, KVH,
-                       sl2);
+    auto go = [&](auto kern) {   // heads fastest: the heavy tiles of every head go first
+        const uint32_t qt = 32 * form.wph;
+        hipLaunchKernelGGL(kern, dim3(H, (S + qt - 1) / qt), dim3(64 * form.np * form.wph), 0, st, q, ldq, qhs, k, v, ldkv,
+                           kvhs, out, ldo, ohs, S, H, KVH, sl2);
+    };
+    if (form.np == 4) {
+        if (form.wph == 2) go(causal ? attn_prefill_kernel<true, 2, 4> : attn_prefill_kernel<false, 2, 4>);
+        else go(causal ? attn_prefill_kernel<true, 1, 4> : attn_prefill_kernel<false, 1, 4>);
+    } else if (form.wph == 4) {
+        go(causal ? attn_prefill_kernel<true, 4, 2> : attn_prefill_kernel<false, 4, 2>);
+    } else if (form.wph == 2) {
+        go(causal ? attn_prefill_kernel<true, 2, 2> : attn_prefill_kernel<false, 2, 2>);
+    } else {
+        go(causal ? attn_prefill_kernel<true, 1, 2> : attn_prefill_kernel<false, 1, 2>);
+    }
     return hipGetLastError();
 }
 

@@ -405,6 +405,28 @@ def test_attn_prefill_tile_sizes(lib, oracle, torch_dev, causal):
     assert_close(big, ref, what=f"128-query tiles causal={causal}")
 
 
+@pytest.mark.parametrize("S,H,causal", [(513, 8, True), (600, 16, True), (577, 8, False), (700, 16, False), (641, 48, True),
+                                        (769, 32, False)])
+def test_attn_prefill_four_parts(lib, oracle, torch_dev, S, H, causal):
+    """Past 512 tokens, grids of up to one workgroup per CU split a tile's key stages over
+    four parts (32-query tiles at 8 heads, 64-query at 16; 9 stages of 513..576 tokens leave
+    the last part empty, and one key in the last stage at 513, 577); larger grids (48 heads,
+    32 without a mask) take two parts. Keys grow along S, so that late stages move the
+    reference max and the parts' maxima differ."""
+    import torch
+    rng = np.random.default_rng(S)
+    KVH, hd = 8, 128
+    q, k, v = normal_f16(rng, S, H, hd), normal_f16(rng, S, KVH, hd), normal_f16(rng, S, KVH, hd)
+    k = (k.astype(np.float32) * (1.0 + 3.0 * np.arange(S, dtype=np.float32) / S)[:, None, None]).astype(np.float16)
+    out = torch.full((S + 1, H, hd), 7.0, dtype=torch.float16, device=torch_dev)
+    assert lib.gehtp_attn_prefill(ptr(to_dev(q, torch_dev)), ptr(to_dev(k, torch_dev)), ptr(to_dev(v, torch_dev)),
+                                  ptr(out), S, H, KVH, hd, SCALE, int(causal), stream_ptr()) == 0
+    _sync()
+    got = from_dev(out)
+    assert_close(got[:S], oracle.attn_prefill(q, k, v, SCALE, causal, threads=8), what=f"attn S={S} H={H}")
+    assert (got[S] == 7.0).all()   # nothing written past the last query
+
+
 @pytest.mark.parametrize("n_kv,H,KVH", [(4096, 16, 8), (77, 32, 8), (1, 16, 8)])
 def test_attn_decode(lib, oracle, torch_dev, n_kv, H, KVH):
     """Config 3 decode: batch 1 over a KV cache of n_kv tokens in the reference ring layout."""
