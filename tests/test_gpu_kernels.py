@@ -455,6 +455,34 @@ def test_attn_decode(lib, oracle, torch_dev, n_kv, H, KVH):
     assert_close(from_dev(out), ref, what=f"decode n_kv={n_kv}")
 
 
+@pytest.mark.parametrize("n_kv,H", [(4096 + 1, 16), (4096 + 64 * 9, 8), (8192, 32), (8192 + 64 * 7 + 5, 16), (12300, 16)])
+def test_attn_decode_merge_rounds(lib, oracle, torch_dev, n_kv, H):
+    """The merge takes a head's chunks of 64 keys in rounds of 64 (8 thread groups x 8
+    records): contexts that end one key, nine chunks or 7 chunks and 5 keys into a round, or
+    on its edge. Keys grow along the context, so that later rounds move the maximum."""
+    import torch
+    rng = np.random.default_rng(n_kv)
+    KVH, hd = 8, 128
+    kv_elems = KVH * hd
+    state_bytes = n_kv * kv_elems * 4
+    ring = oracle.KVRing(state_bytes, kv_elems)
+    ks, vs = normal_f16(rng, n_kv, kv_elems), normal_f16(rng, n_kv, kv_elems)
+    ks = (ks.astype(np.float32) * (1.0 + np.arange(n_kv, dtype=np.float32) / n_kv)[:, None]).astype(np.float16)
+    for t in range(n_kv):
+        ring.append(ks[t], vs[t])
+    q = normal_f16(rng, H, hd)
+    ring_d = torch.zeros(state_bytes, dtype=torch.uint8, device=torch_dev)
+    assert lib.gehtp_kv_append(ptr(ring_d), state_bytes, ptr(to_dev(ks, torch_dev)), ptr(to_dev(vs, torch_dev)),
+                               kv_elems, n_kv, 0, stream_ptr()) == 0
+    wf = lib.gehtp_attn_decode_work_floats(n_kv, H, hd)
+    work = torch.zeros(wf, dtype=torch.float32, device=torch_dev)
+    out = torch.empty((H, hd), dtype=torch.float16, device=torch_dev)
+    assert lib.gehtp_attn_decode(ptr(to_dev(q, torch_dev)), ptr(ring_d), state_bytes, ptr(out), n_kv, H, KVH, hd,
+                                 SCALE, ptr(work), wf, stream_ptr()) == 0
+    _sync()
+    assert_close(from_dev(out), ring.attn_decode(q, n_kv, H, KVH, hd, SCALE), what=f"decode n_kv={n_kv}")
+
+
 def test_decode_matches_prefill_last_row(lib, torch_dev):
     """Decode of token t over keys [0, t] equals row t of the causal prefill (reference's
     decode==prefill gate, scripts/judge_logits.py: cos >= 0.9999)."""
