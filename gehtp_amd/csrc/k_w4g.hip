@@ -26,7 +26,7 @@ namespace gehtp {
 namespace {
 
 // ---------------------------------------------------------------------------
-// GEMV (M <= 4). A weight row is S = K/32 slices of 16 bytes (32 weights, half a
+// GEMV (M = 1, 2). A weight row is S = K/32 slices of 16 bytes (32 weights, half a
 // scale group). P = S threads share a row, each owning one slice; R = nthreads/P rows
 // are processed per pass and a workgroup runs np passes over its R*np contiguous rows.
 // A thread's activation slice stays in registers (pair order) for the whole kernel,

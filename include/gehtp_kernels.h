@@ -26,7 +26,7 @@ extern "C" {
 #define GEHTP_E2BIG (-7)   /* request larger than a fixed-size scratch */
 
 /* y[M, ldy] = x[M, ldx] . dequant(W)^T, W4G int4 group-64 (OP_MATMUL_W4G_F16):
- * M <= 4 runs the GEMV, larger M the MFMA GEMM. Mirrors exec_matmul_f16's scalar
+ * M <= 2 runs the GEMV, larger M an MFMA GEMM (its few-row form up to 32). Mirrors exec_matmul_f16's scalar
  * arithmetic (oplist_exec.c:1802-1811) on dequant(W) = fp16(q*s) with fp32
  * accumulation (summation order differs).
  * K % 64 == 0, ldx % 8 == 0, x and wq 16-byte aligned. */
