@@ -137,15 +137,17 @@ __device__ __forceinline__ uint32_t xcd_tile(uint32_t x, uint32_t n) {
 // k = (64 / CW) wave + lane / CW, so a load instruction covers 64 / CW rows, and every lane
 // keeps 4 or 8 rows in flight (16 waves: 128 KiB per workgroup at 8); the k lanes' sums meet
 // by DPP and row swaps, the waves' in LDS. Needs N >= 8 (the last chunk is moved back to
-// end at column N; columns computed twice get the same value). CW = 4 where that grid
-// covers the CUs, else 2 (twice the workgroups; 1 x 2560 x 9728: 20 / 17.9 us).
+// end at column N; columns computed twice get the same value), so a window of fewer columns
+// is computed in one of 8 and only columns [lo, lo + cnt) of it are stored. CW = 4 where that
+// grid covers the CUs, else 2 (twice the workgroups; 1 x 2560 x 9728: 20 / 17.9 us).
 // Bound: w's bytes; one thread per column walked K serially on N / 256 workgroups before
 // (1 x 3072 x 1024: 131.9 -> 4.2 us a call; 1 x 2560 x 9728: 2.8 TB/s).
 template <int MR, int CW>
 __global__ __launch_bounds__(1024) void gemv_kn_kernel(const __half* __restrict__ a,
                                                        const __half* __restrict__ w,
                                                        __half* __restrict__ y, uint32_t K,
-                                                       uint32_t N_full, uint32_t n0, uint32_t N, int t0) {
+                                                       uint32_t N_full, uint32_t n0, uint32_t N, uint32_t lo,
+                                                       uint32_t cnt, int t0) {
     constexpr int UMAX = MR <= 2 ? 8 : 4;              // rows in flight per lane
     constexpr uint32_t KR = 64 / CW, PASS = 16 * KR;   // k rows per wave and per workgroup pass
     __shared__ __align__(16) float red[16][MR][8 * CW];
@@ -220,7 +222,7 @@ __global__ __launch_bounds__(1024) void gemv_kn_kernel(const __half* __restrict_
 #pragma unroll
         for (int i = 0; i < 16; ++i) v += red[i][m][j];
         const uint32_t col = min(c0 + (j & ~7u), N - 8) + (j & 7);
-        y[((size_t)bb * MR + m) * N_full + n0 + col] = __float2half(v);
+        if (col - lo < cnt) y[((size_t)bb * MR + m) * N_full + n0 + col] = __float2half(v);
     }
 }
 
@@ -492,11 +494,15 @@ hipError_t gemm_f16_launch(const __half* a, const __half* w, __half* y, uint32_t
         return hipGetLastError();
     };
     const size_t cus = (size_t)device_cu_count();
-    // Tile by the grid's rounds: a round of one workgroup per CU took 2.4 / 4.2 / 11.5 us per
-    // 1024 of K with 32 / 64 / 128-square tiles. Measured with the three, us (M x N x K):
-    // 256 x 1024 x 1024 4.5 / 6.9 / 15.1; 512 x 3072 x 1024 17.0 / 11.0 / 15.7; 117 x 3760 x 3072
-    // 31 / 15.7 / 36; 1024 x 4096 x 4096 194 / 64 / 49.
-    auto cost = [&](size_t b, double us) { return us * (double)(((M + b - 1) / b * ((N + b - 1) / b) * Bn + cus - 1) / cus); };
+    // Tile by the rounds of the whole product's grid, not the window's: the 32-square tile sums
+    // K in another order than the others, and a SPLIT chunk has the whole product's bits. A
+    // round of one workgroup per CU took 2.4 / 4.2 / 11.5 us per 1024 of K with 32 / 64 /
+    // 128-square tiles. Measured with the three, us (M x N x K): 256 x 1024 x 1024 4.5 / 6.9 /
+    // 15.1; 512 x 3072 x 1024 17.0 / 11.0 / 15.7; 117 x 3760 x 3072 31 / 15.7 / 36;
+    // 1024 x 4096 x 4096 194 / 64 / 49.
+    auto cost = [&](size_t b, double us) {
+        return us * (double)(((M + b - 1) / b * ((N_full + b - 1) / b) * Bn + cus - 1) / cus);
+    };
     const double c32 = cost(32, 2.4), c64 = cost(64, 4.2), c128 = cost(128, 11.5);
     const int t = c128 < c64 && c128 < c32 ? 128 : c64 < c32 ? 64 : 32;
     if (t == 128) return go(gemm_f16_kernel<128, 128, 2, 2, 1, 64, 2, AK, BKM>, 128, 128, 256);
@@ -536,18 +542,21 @@ hipError_t launch_matmul_f16(const __half* a, const __half* w, __half* y, uint32
         }
         return hipGetLastError();
     }
-    if (M <= 4 && !t1 && N >= 8) {
+    if (M <= 4 && !t1 && N_full >= 8) {
         const int ta = t0 && !batched;
+        const uint32_t nw = std::max(N, 8u), n0w = std::min(n0, N_full - nw);   // window computed
         auto go = [&](auto kern, uint32_t cols) {
-            hipLaunchKernelGGL(kern, dim3((N + cols - 1) / cols, Bn), dim3(1024), 0, st, a, w, y, K, N_full, n0, N, ta);
+            hipLaunchKernelGGL(kern, dim3((nw + cols - 1) / cols, Bn), dim3(1024), 0, st, a, w, y, K, N_full, n0w, nw,
+                               n0 - n0w, N, ta);
             return hipGetLastError();
         };
         // 16-column workgroups where 32-column ones leave CUs idle and K fills their passes; rows
         // off 16-byte boundaries make 32-byte pieces cross lines, which only long K makes up for
         // (1 x 3073 x 1024: 4.8 us with 32 columns, 6.9 with 16; 1 x 2561 x 9728: 26.0 / 24.0;
-        // 1 x 2560 x 9728: 20 / 18).
-        const bool al = N_full % 8 == 0 && reinterpret_cast<uintptr_t>(w + n0) % 16 == 0;
-        const bool wide = (size_t)((N + 31) / 32) * Bn >= (size_t)device_cu_count() || K < (al ? 1024u : 2048u);
+        // 1 x 2560 x 9728: 20 / 18). The two order K differently, so the whole product decides
+        // here too, not the window.
+        const bool al = N_full % 8 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
+        const bool wide = (size_t)((N_full + 31) / 32) * Bn >= (size_t)device_cu_count() || K < (al ? 1024u : 2048u);
         switch (M) {
         case 1: return wide ? go(gemv_kn_kernel<1, 4>, 32) : go(gemv_kn_kernel<1, 2>, 16);
         case 2: return wide ? go(gemv_kn_kernel<2, 4>, 32) : go(gemv_kn_kernel<2, 2>, 16);

@@ -184,3 +184,30 @@ def test_matmul_f16_split_chunks(engine, oracle, M, K, N, t1):
     assert np.array_equal(whole.view(np.uint16), split.view(np.uint16))
     want = oracle.matmul_f16(a, w, M, K, N, flags=flags)
     assert_close(split.reshape(M, N), want.reshape(M, N), what=f"split M{M} K{K} N{N}")
+
+
+@pytest.mark.parametrize("M,K,N,cuts,t1", [
+    (128, 1024, 3072, (1024, 2048), False), (128, 1024, 3072, (1024, 2048), True),   # 64-square whole, 32-square by chunk width
+    (1024, 256, 4096, (512,), False),                                                # 128-square whole
+    (1, 1024, 8200, (2720, 5440), False),                                            # 32-column GEMV whole, 16-column by chunk width
+    (3, 1100, 72, (13, 18, 19, 65), False),                                          # GEMV chunks of 1, 5 and 7 columns, off alignment
+    (70, 300, 37, (3, 8, 30), False),                                                # GEMM chunks of rows shorter than a load
+])
+def test_matmul_f16_split_across_forms(engine, oracle, M, K, N, cuts, t1):
+    """Opcode 35 where the chunk's own width would choose another tile or column group than
+    the whole product's: the order in which K is summed depends on neither, so the chunks
+    are byte-identical to opcode 24."""
+    rng = np.random.default_rng(M + N)
+    a = (normal_f16(rng, M, K) * np.float16(0.25)).astype(np.float16)
+    w = ((normal_f16(rng, N, K) if t1 else normal_f16(rng, K, N)) * np.float16(0.25)).astype(np.float16)
+    flags, edges = (2 if t1 else 0), [0, *cuts, N]
+    bb = BlobBuilder()
+    sa, sw = bb.add_slot(a), bb.add_slot(w)
+    t_whole, t_split = bb.temp(), bb.temp()
+    bb.op(OP.MATMUL_F16, bb.slot_ref(sa), bb.slot_ref(sw), t_whole, M, K, N, flags)
+    for c0, c1 in zip(edges[:-1], edges[1:]):
+        bb.op(OP.MATMUL_F16_SPLIT, bb.slot_ref(sa), bb.slot_ref(sw), t_split, M, K, N, c0, c1 - c0, flags)
+    out = _run(engine, bb, {"w": t_whole, "s": t_split})
+    whole, split = out["w"][:M * N], out["s"][:M * N]
+    assert np.array_equal(whole.view(np.uint16), split.view(np.uint16))
+    assert_close(split.reshape(M, N), oracle.matmul_f16(a, w, M, K, N, flags=flags).reshape(M, N), what=f"M{M} K{K} N{N}")
