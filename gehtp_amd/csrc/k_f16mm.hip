@@ -4,7 +4,8 @@
 //
 //   M <= 4, t1:   GEMV, one wavefront per output column n streaming w's row n (the
 //                 lm_head path); activations staged once per workgroup in LDS.
-//   M <= 4, !t1:  GEMV over columns: 8 columns per lane, K split over a workgroup.
+//   M <= 4, !t1:  GEMV over columns: 8 columns per lane, K split over a workgroup; for short
+//                 K one column per thread.
 //   otherwise:    MFMA 32x32x16 tiles (any shape, flags, alignment).
 #include "dev_reduce.h"
 #include "kernels.h"
@@ -224,6 +225,30 @@ __global__ __launch_bounds__(1024) void gemv_kn_kernel(const __half* __restrict_
         const uint32_t col = min(c0 + (j & ~7u), N - 8) + (j & 7);
         if (col - lo < cnt) y[((size_t)bb * MR + m) * N_full + n0 + col] = __float2half(v);
     }
+}
+
+// The same for short K: one column per thread, K in order.
+template <int MR>
+__global__ __launch_bounds__(256) void gemv_col_kernel(const __half* __restrict__ a, const __half* __restrict__ w,
+                                                       __half* __restrict__ y, uint32_t K, uint32_t N_full, uint32_t n0,
+                                                       uint32_t N, int t0) {
+    const uint32_t bb = blockIdx.y, n = blockIdx.x * 256 + threadIdx.x;
+    if (n >= N) return;
+    const __half* ab = a + (size_t)bb * MR * K;
+    const __half* wb = w + (size_t)bb * K * N_full + n0 + n;
+    const uint32_t as = t0 ? MR : 1u, am = t0 ? 1u : K;   // strides of a along k and m
+    float acc[MR];
+#pragma unroll
+    for (int m = 0; m < MR; ++m) acc[m] = 0.0f;
+#pragma unroll 8
+    for (uint32_t k = 0; k < K; ++k) {
+        const float wv = __half2float(wb[(size_t)k * N_full]);
+#pragma unroll
+        for (int m = 0; m < MR; ++m)
+            acc[m] = __builtin_fmaf(__half2float(ab[(size_t)k * as + (size_t)m * am]), wv, acc[m]);
+    }
+#pragma unroll
+    for (int m = 0; m < MR; ++m) y[((size_t)bb * MR + m) * N_full + n0 + n] = __float2half(acc[m]);
 }
 
 // --- MFMA GEMM ---------------------------------------------------------------------
@@ -493,20 +518,25 @@ hipError_t gemm_f16_launch(const __half* a, const __half* w, __half* y, uint32_t
                            n0, N);
         return hipGetLastError();
     };
+    // K of one short step: the same order as the 64- and 128-square tiles, half their staging
+    // (5 x 32768 x 4 with steps of 64: 4.1 us, now 3.4).
+    if (K <= 32) return go(gemm_f16_kernel<64, 64, 2, 2, 1, 32, 2, AK, BKM>, 64, 64, 256);
     const size_t cus = (size_t)device_cu_count();
-    // Tile by the rounds of the whole product's grid, not the window's: the 32-square tile sums
-    // K in another order than the others, and a SPLIT chunk has the whole product's bits. A
-    // round of one workgroup per CU took 2.4 / 4.2 / 11.5 us per 1024 of K with 32 / 64 /
-    // 128-square tiles. Measured with the three, us (M x N x K): 256 x 1024 x 1024 4.5 / 6.9 /
-    // 15.1; 512 x 3072 x 1024 17.0 / 11.0 / 15.7; 117 x 3760 x 3072 31 / 15.7 / 36;
-    // 1024 x 4096 x 4096 194 / 64 / 49.
-    auto cost = [&](size_t b, double us) {
-        return us * (double)(((M + b - 1) / b * ((N_full + b - 1) / b) * Bn + cus - 1) / cus);
+    // Tile by the grid's rounds. A round of one workgroup per CU took 2.4 / 4.2 / 11.5 us per
+    // 1024 of K with 32 / 64 / 128-square tiles. Measured with the three, us (M x N x K):
+    // 256 x 1024 x 1024 4.5 / 6.9 / 15.1; 512 x 3072 x 1024 17.0 / 11.0 / 15.7; 117 x 3760 x 3072
+    // 31 / 15.7 / 36; 1024 x 4096 x 4096 194 / 64 / 49.
+    // The 32-square tile sums K in another order than the other two, so whether it runs is the
+    // whole product's choice and not a window's (128 x 1024 of 3072 x 1024: 4.8 us with it,
+    // 7.3 without): a SPLIT chunk has the whole product's bits.
+    auto cost = [&](size_t b, uint32_t n, double us) {
+        return us * (double)(((M + b - 1) / b * ((n + b - 1) / b) * Bn + cus - 1) / cus);
     };
-    const double c32 = cost(32, 2.4), c64 = cost(64, 4.2), c128 = cost(128, 11.5);
-    const int t = c128 < c64 && c128 < c32 ? 128 : c64 < c32 ? 64 : 32;
-    if (t == 128) return go(gemm_f16_kernel<128, 128, 2, 2, 1, 64, 2, AK, BKM>, 128, 128, 256);
-    if (t == 64) return go(gemm_f16_kernel<64, 64, 2, 2, 1, 64, 4, AK, BKM>, 64, 64, 256);
+    if (cost(64, N_full, 4.2) < cost(32, N_full, 2.4) || cost(128, N_full, 11.5) < cost(32, N_full, 2.4)) {
+        if (cost(128, N, 11.5) < cost(64, N, 4.2))
+            return go(gemm_f16_kernel<128, 128, 2, 2, 1, 64, 2, AK, BKM>, 128, 128, 256);
+        return go(gemm_f16_kernel<64, 64, 2, 2, 1, 64, 4, AK, BKM>, 64, 64, 256);
+    }
     return go(gemm_f16_kernel<32, 32, 1, 1, 8, 128, 4, AK, BKM>, 32, 32, 512);
 }
 
@@ -542,8 +572,20 @@ hipError_t launch_matmul_f16(const __half* a, const __half* w, __half* y, uint32
         }
         return hipGetLastError();
     }
+    const int ta = t0 && !batched;
+    // Short K: a workgroup of the split form costs the same whatever K, a column per thread about
+    // 0.1 us per k and row of a. Measured, us, split / one column per thread: 1 x 4096 x 8 3.1 /
+    // 2.7, x 16 3.1 / 3.6; 4 x 4096 x 12 6.1 / 6.1; 1 x 32768 x 32 5.9 / 5.4, 4 x 32768 x 48 19.5 /
+    // 18.7 (1, 2 and 4 split workgroups per CU).
+    const uint64_t per_cu = ((uint64_t)(N_full + 31) / 32 * Bn + device_cu_count() - 1) / device_cu_count();
+    if (M <= 4 && !t1 && K <= std::min<uint64_t>(128, 13 + (M % 2 ? 7 : 11) * (per_cu - 1))) {
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3((N + 255) / 256, Bn), dim3(256), 0, st, a, w, y, K, N_full, n0, N, ta);
+            return hipGetLastError();
+        };
+        return M == 1 ? go(gemv_col_kernel<1>) : M == 2 ? go(gemv_col_kernel<2>) : M == 3 ? go(gemv_col_kernel<3>) : go(gemv_col_kernel<4>);
+    }
     if (M <= 4 && !t1 && N_full >= 8) {
-        const int ta = t0 && !batched;
         const uint32_t nw = std::max(N, 8u), n0w = std::min(n0, N_full - nw);   // window computed
         auto go = [&](auto kern, uint32_t cols) {
             hipLaunchKernelGGL(kern, dim3((nw + cols - 1) / cols, Bn), dim3(1024), 0, st, a, w, y, K, N_full, n0w, nw,

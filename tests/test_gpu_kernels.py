@@ -793,7 +793,10 @@ def test_attn_decode_qkv_matches_unfused(lib, oracle, torch_dev, H, KVH, pos0):
 @pytest.mark.parametrize("M,K,N,Bn", [(1, 1024, 48, 1), (2, 2050, 33, 1), (3, 700, 9, 1), (4, 2048, 8, 2), (1, 260, 8200, 1),
                                       (1, 3, 7, 1), (5, 7, 5, 1), (33, 128, 32, 1), (5, 641, 31, 1), (31, 1025, 45, 3),
                                       (64, 200, 1000, 8), (65, 1022, 4100, 1), (700, 131, 1300, 1), (1000, 64, 70, 40),
-                                      (1030, 72, 8200, 1), (1030, 79, 8201, 1), (2050, 66, 4097, 2)])
+                                      (1030, 72, 8200, 1), (1030, 79, 8201, 1), (2050, 66, 4097, 2),
+                                      # short K: one column per thread, and 64-square tiles in steps of 32
+                                      (1, 1, 1, 1), (2, 13, 300, 1), (3, 5, 7, 1), (4, 24, 8193, 2), (1, 128, 131080, 1),
+                                      (5, 32, 65, 1), (65, 31, 63, 3), (130, 9, 9, 1), (33, 33, 64, 1)])
 def test_matmul_f16_tiles_and_edges(lib, torch_dev, M, K, N, Bn):
     """The tiles (32, 64 and 128 square by the grid's size; 16- and 32-column GEMV
     workgroups), their remainders in M, N and K, rows off every alignment, rows of fewer
