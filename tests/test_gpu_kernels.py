@@ -794,6 +794,8 @@ def test_attn_decode_qkv_matches_unfused(lib, oracle, torch_dev, H, KVH, pos0):
                                       (1, 3, 7, 1), (5, 7, 5, 1), (33, 128, 32, 1), (5, 641, 31, 1), (31, 1025, 45, 3),
                                       (64, 200, 1000, 8), (65, 1022, 4100, 1), (700, 131, 1300, 1), (1000, 64, 70, 40),
                                       (1030, 72, 8200, 1), (1030, 79, 8201, 1), (2050, 66, 4097, 2),
+                                      # [K, N] GEMV of 1 or 2 rows: whole 8-row passes, then four, then the edge
+                                      (1, 9728, 2560, 1), (2, 4096 + 2048 + 37, 72, 1), (1, 2048 + 1024 + 5, 8200, 1),
                                       # short K: one column per thread, and 64-square tiles in steps of 32
                                       (1, 1, 1, 1), (2, 13, 300, 1), (3, 5, 7, 1), (4, 24, 8193, 2), (1, 128, 131080, 1),
                                       (5, 32, 65, 1), (65, 31, 63, 3), (130, 9, 9, 1), (33, 33, 64, 1)])
@@ -928,3 +930,34 @@ def test_softmax_row_per_wave(lib, torch_dev, rows, n):
         ref = torch.softmax(x.double(), -1)
         err = (got - ref).abs()
         assert (err <= ref * (2 ** -10 + (n + 16) * 2 ** -24) + 2 ** -24).all(), (off, float(err.max()))
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 9728, 264), (1, 12, 264), (2, 700, 1032), (4, 1100, 40), (3, 3100, 8200)])
+def test_matmul_f16_gemv_special_values(lib, torch_dev, M, K, N):
+    """The [K, N] GEMVs with a NaN, an infinity of each sign and 65504s in single columns of w
+    (the first and last row of K, and inside): only those columns show them, the others keep
+    their bits; an infinity in a's row reaches that row alone."""
+    import torch
+    g = torch.Generator(device=torch_dev).manual_seed(M + K + N)
+    a = torch.randn((M, K), device=torch_dev, generator=g).half()
+    w = (torch.randn((K, N), device=torch_dev, generator=g) * K ** -0.5).half()
+
+    def run(a, w):
+        y = torch.empty((M, N), dtype=torch.float16, device=torch_dev)
+        assert lib.gehtp_matmul_f16(ptr(a), ptr(w), ptr(y), M, K, N, 0, N, 0, stream_ptr()) == 0
+        _sync()
+        return y
+
+    clean, hot = run(a, w), w.clone()
+    cols = [0, 9, N // 2, N - 1]
+    hot[K - 1, cols[0]], hot[0, cols[1]], hot[K // 2, cols[2]], hot[:, cols[3]] = float("nan"), float("inf"), -float("inf"), 65504
+    got = run(a, hot)
+    keep = [j for j in range(N) if j not in cols]
+    assert torch.equal(got[:, keep].view(torch.int16), clean[:, keep].view(torch.int16))
+    ref = (a.double() @ hot.double()).half()   # an overflow of the fp16 result is an infinity
+    for j in cols:
+        assert torch.equal(torch.isnan(got[:, j]), torch.isnan(ref[:, j])) and torch.equal(torch.isinf(got[:, j]), torch.isinf(ref[:, j]))
+    a2 = a.clone()
+    a2[M - 1, K - 1] = float("inf")
+    rows = run(a2, w)
+    assert torch.equal(rows[:M - 1].view(torch.int16), clean[:M - 1].view(torch.int16)) and not torch.isfinite(rows[M - 1]).any()
