@@ -1325,13 +1325,17 @@ static hipError_t launch_skinny(const __half* a, uint32_t lda, const uint8_t* wq
                            epi.res, epi.ldr, epi.swiglu ? 1 : 0, epi.gamma);
         return hipGetLastError();
     };
-    // Column tiles per workgroup: the fewest on the busiest CU, then the widest (A is
-    // staged once per workgroup). M = 8, us at NT = 1 / 2 / 3 / 5 (8 waves, 4 from NT = 3):
-    // 2560 x 9728 9.5 / 14.1 / 19.8 / 29.6, 6144 x 2560 5.5 / 5.3 / 6.2 / 8.6, 19456 x 2560
-    // 15.5 / 14.2 / 13.1 / 12.5 (1216 tiles: 5 on the busiest CU with 1 or 5, 6 with 2 or 3).
+    // Column tiles per workgroup (8 waves for 1 or 2, 4 for 3 or 5): the fewest on the busiest
+    // CU, then the widest (A is staged once per workgroup). What an 8-wave workgroup costs beside
+    // its tiles counts as a quarter of one (half of one at 17 to 32 rows, a fifth for few rows of
+    // long K). M = 8, us at 1 / 2 / 3 / 5: 2560 x 9728 9.5 / 14.1 / 19.8 / 29.6, 6144 x 2560 5.5 /
+    // 5.3 / 6.2 / 8.6, 19456 x 2560 15.5 / 14.2 / 13.1 / 12.5 (1216 tiles: 5 on the busiest CU
+    // with 1 or 5, 6 with 2 or 3), 151936 x 1024 37.4 / 35.8 / 31.0 / 31.2; M = 32, 151936 x 1024
+    // 79.7 / 72.6 / 45.8 / 44.0 (38 / 38 / 39 / 40 on the busiest; 50.1 on 128-column tiles).
+    const uint32_t wide_wg = M > 16 ? 10u : M <= 8 && K >= 4096 ? 4u : 5u;   // in twentieths of a tile
     uint32_t nt = 1, best = ~0u;
     for (uint32_t c : {1u, 2u, 3u, 5u}) {
-        const uint32_t busiest = ((tiles + c - 1) / c + cu - 1) / cu * c;
+        const uint32_t busiest = ((tiles + c - 1) / c + cu - 1) / cu * (20 * c + (c < 3 ? wide_wg : 0u));
         if (busiest <= best) { best = busiest; nt = c; }
     }
     auto rows = [&](auto ar, auto norm) {

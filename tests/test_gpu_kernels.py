@@ -961,3 +961,33 @@ def test_matmul_f16_gemv_special_values(lib, torch_dev, M, K, N):
     a2[M - 1, K - 1] = float("inf")
     rows = run(a2, w)
     assert torch.equal(rows[:M - 1].view(torch.int16), clean[:M - 1].view(torch.int16)) and not torch.isfinite(rows[M - 1]).any()
+
+
+@pytest.mark.parametrize("M,N,K,mode,norm", [
+    (20, 32784, 320, 0, False), (5, 33000, 192, 1, False), (2, 65552, 128, 0, True)])   # 3 column tiles where 2 would do
+def test_w4g_few_rows_forms(lib, oracle, torch_dev, M, N, K, mode, norm):
+    """Up to 32 rows where the rules change kernels on 256 CUs: the GEMV, the few-row GEMM (by
+    its column tiles per workgroup) and the 128-column tiles, with and without their K parts.
+    Against the oracle's RMSNorm, linear and SwiGLU, and within fp32 sums of each other with
+    and without a workspace."""
+    import torch
+    rng = np.random.default_rng(M + N + K)
+    n_out = N // 2 if mode else N
+    _, wq, ws = w4g_weights(rng, N, K)
+    x = normal_f16(rng, M, K) * np.float16(0.25)
+    gamma = (rng.uniform(0.8, 1.2, K) * 0.25).astype(np.float16)
+    xd, wd, sd, gd = (to_dev(v, torch_dev) for v in (x, wq, ws, gamma))
+    xr = oracle.rmsnorm2(x, gamma, np.zeros(K, np.float16)) if norm else x
+    acc = oracle.matmul_w4g(xr, wq, ws, threads=8)
+    ref = oracle.binary(oracle.unary(acc[:, 0::2].copy(), 12), acc[:, 1::2].copy(), 2) if mode else acc
+    nb = lib.gehtp_w4g_split_bytes(M, N, K)
+    assert (nb > 0) == ((M, N) in ((24, 14336), (32, 8448)))
+    for work in (None, torch.empty(nb // 4, dtype=torch.float32, device=torch_dev)) if nb else (None,):
+        y = torch.full((M + 1, n_out), 7.0, dtype=torch.float16, device=torch_dev)
+        assert lib.gehtp_w4g_fused_ws(ptr(xd), K, ptr(wd), ptr(sd), ptr(y), n_out, M, N, K, ptr(gd) if norm else None, None,
+                                      n_out, mode, ptr(work) if work is not None else None, nb if work is not None else 0,
+                                      stream_ptr()) == 0
+        _sync()
+        got = from_dev(y)
+        assert (got[M] == 7).all()
+        assert_close(got[:M], ref, what=f"{M}x{N}x{K} mode={mode} norm={norm} work={work is not None}")
