@@ -62,7 +62,8 @@ extern "C" {
 int gehtp_w4g_gemv(const void* x, uint32_t ldx, const void* wq, const void* ws, void* y, uint32_t ldy,
                    uint32_t M, uint32_t N, uint32_t K, void* stream) {
     if (!w4g_args_ok(x, ldx, wq, ws, y, ldy, N, K) || M > kW4gGemvMaxM) return GEHTP_EINVAL;
-    return rc(launch_w4g_gemv(H(x), ldx, static_cast<const uint8_t*>(wq), H(ws), Hm(y), ldy, M, N, K, S(stream)));
+    return rc(launch_w4g_gemv(H(x), ldx, static_cast<const uint8_t*>(wq), H(ws), Hm(y), ldy, M, N, K, S(stream),
+                              W4gEpilogue(), /*gemv_only=*/true));
 }
 
 int gehtp_w4g_gemm(const void* x, uint32_t ldx, const void* wq, const void* ws, void* y, uint32_t ldy,
@@ -73,8 +74,9 @@ int gehtp_w4g_gemm(const void* x, uint32_t ldx, const void* wq, const void* ws, 
 
 int gehtp_w4g_matmul(const void* x, uint32_t ldx, const void* wq, const void* ws, void* y, uint32_t ldy,
                      uint32_t M, uint32_t N, uint32_t K, void* stream) {
-    return M <= kW4gGemvMaxM ? gehtp_w4g_gemv(x, ldx, wq, ws, y, ldy, M, N, K, stream)
-                             : gehtp_w4g_gemm(x, ldx, wq, ws, y, ldy, M, N, K, stream);
+    if (M > kW4gGemvMaxM) return gehtp_w4g_gemm(x, ldx, wq, ws, y, ldy, M, N, K, stream);
+    if (!w4g_args_ok(x, ldx, wq, ws, y, ldy, N, K)) return GEHTP_EINVAL;
+    return rc(launch_w4g_gemv(H(x), ldx, static_cast<const uint8_t*>(wq), H(ws), Hm(y), ldy, M, N, K, S(stream)));
 }
 
 int gehtp_w4g_fused(const void* x, uint32_t ldx, const void* wq, const void* ws, void* y, uint32_t ldy,

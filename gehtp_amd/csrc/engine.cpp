@@ -1196,7 +1196,7 @@ int op_w4g_fused(Ctx& cx) {
     // do few rows, whose GEMM is another kernel (M = 8, N 4096, K 1024: 3.4 us and the op's 4,
     // against 6.8 and the table's 4).
     const wt_op* rx = cx.op + 1;
-    if (fusion_on() && !w4g_gemm_skinny(M) && !swiglu && !res && ldy == N && (uint32_t)(rx - cx.b->ops) < g_run_end &&
+    if (fusion_on() && !w4g_gemm_skinny(M, N, K) && !swiglu && !res && ldy == N && (uint32_t)(rx - cx.b->ops) < g_run_end &&
         rx->opcode == OP_QK_ROPE_KV_F16 && rx->n_args >= 12 && rx->args[0] == A(3) && rx->args[5] == M &&
         rx->args[8] == 128 && (uint64_t)(rx->args[6] + 2ull * rx->args[7]) * 128u == N) {
         QkRope r;

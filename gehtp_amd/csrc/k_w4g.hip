@@ -703,7 +703,7 @@ __global__ __launch_bounds__(256, 3) void w4g_gemm_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// GEMM of few rows (M <= 32): weights stream once, so a tile is 16 NT columns of all M rows
+// GEMM of few rows (M <= 32, w4g_gemm_skinny): weights stream once, so a tile is 16 NT columns of all M rows
 // (AR >= M of them staged; with NORM, M <= 4, normalized as they are staged) and K is split over the workgroup's WV waves in contiguous ranges
 // of 128-deep blocks, their sums added in LDS in wave order; no workspace, one launch. On
 // v_mfma_f32_16x16x32_f16 lane l supplies column (A row) l % 16 and, with j = l / 16, the k's
@@ -1351,9 +1351,28 @@ static hipError_t launch_skinny(const __half* a, uint32_t lda, const uint8_t* wq
                    : rows(std::integral_constant<int, 32>{}, std::false_type{});
 }
 
+// Whether the GEMV takes M rows it has a plan for, or w4g_skinny_kernel does: three or four
+// rows, and two with the RMSNorm (whose prologue the GEMV repeats in every workgroup, for all
+// rows at once), mostly run faster as a GEMM. us, GEMV against GEMM, M = 2 / 3 / 4: 19456 x 2560
+// with the RMSNorm 18.2 / 28.6 / 42.9 against 13.3 / 13.4 / 13.4, without 10.5 / 15.3 / 16.8
+// against 11.4 / 11.5 / 11.5; 4096 x 1024 8.2 / 10.5 / 12.3 against 4.3 / 4.3 / 4.4, 3.7 / 4.3 /
+// 4.8 against 3.2 / 3.1 / 3.2. Not where few columns leave long K to few workgroups (M = 3,
+// 1000 x 8192 5.5 against 7.6, with SwiGLU 8.5 / 8.0; M = 4 6.2 / 7.6; M = 2 with the RMSNorm,
+// 256 x 16384 13.2 / 16.4), nor for three rows of large weights whose rows are half waves of
+// slices (65536 x 4096 39.8 / 46.8, 151936 x 3072 72 / 82; 65536 x 2560 39.4 / 31.6).
+static bool gemv_rows(uint32_t M, uint32_t N, uint32_t K, bool norm, bool swiglu) {
+    if (M == 1 || (M == 2 && !norm)) return true;
+    if (norm) return M == 2 && ((N <= 256 && K > 8192) || (N <= 64 && K >= 8192));
+    if (M == 3 && K % 1024 == 0 && K >= 2048 &&
+        (uint64_t)N * K >= (K % 2048 ? 200000000u : K < 8192 ? 150000000u : 75000000u))
+        return true;
+    if (swiglu) return M == 3 && N <= 512 && K >= 8192;
+    return M == 3 ? (N <= 512 && K >= 4096) || (N <= 2048 && K >= 8192) : N <= 1024 && K >= 8192;
+}
+
 hipError_t launch_w4g_gemv(const __half* x, uint32_t ldx, const uint8_t* wq, const __half* ws,
                            __half* y, uint32_t ldy, uint32_t M, uint32_t N, uint32_t K,
-                           hipStream_t st, const W4gEpilogue& epi) {
+                           hipStream_t st, const W4gEpilogue& epi, bool gemv_only) {
     if (M == 0 || N == 0) return hipSuccess;
     if (epi.swiglu && (N & 1)) return hipErrorInvalidValue;
     const GemvPlan pl = gemv_plan(M, K);
@@ -1367,13 +1386,7 @@ hipError_t launch_w4g_gemv(const __half* x, uint32_t ldx, const uint8_t* wq, con
         hipError_t e = hipSuccess;
         if (gemv_rw_launch(GemvRwArgs{x, wq, ws, y, N, K, epi.gamma, epi.res, epi.swiglu ? 1 : 0}, st, &e)) return e;
     }
-    // Three or four rows, and two with the RMSNorm (whose prologue this kernel repeats in
-    // every workgroup, for all rows at once), run faster as a GEMM: us, this kernel against
-    // w4g_skinny_kernel, M = 2 / 3 / 4: 19456 x 2560 with the RMSNorm 18.2 / 28.6 / 42.9
-    // against 13.3 / 13.4 / 13.4, without 10.5 / 15.3 / 16.8 against 11.4 / 11.5 / 11.5;
-    // 4096 x 1024 8.2 / 10.5 / 12.3 against 4.3 / 4.3 / 4.4, 3.7 / 4.3 / 4.8 against
-    // 3.2 / 3.1 / 3.2 (2560 x 9728, M = 2, without: 7.4 against 9.2).
-    if (M >= 3 || (M == 2 && epi.gamma)) return launch_skinny(x, ldx, wq, ws, y, ldy, M, N, K, st, epi);
+    if (!gemv_only && !gemv_rows(M, N, K, epi.gamma != nullptr, epi.swiglu)) return launch_skinny(x, ldx, wq, ws, y, ldy, M, N, K, st, epi);
     // Rows per workgroup: about two workgroups per CU (three when one workgroup holds a
     // single row per pass, as for K = 9728: measured 11 % faster there, slower for the
     // multi-row shapes), partial sums within 32 KiB.
@@ -1408,6 +1421,8 @@ hipError_t launch_w4g_gemv(const __half* x, uint32_t ldx, const uint8_t* wq, con
     switch (M) {
     case 1: return gemv_dispatch<1>(g3, b3, lds, st, A);
     case 2: return gemv_dispatch<2>(g3, b3, lds, st, A);
+    case 3: return gemv_dispatch<3>(g3, b3, lds, st, A);
+    case 4: return gemv_dispatch<4>(g3, b3, lds, st, A);
     default: return hipErrorInvalidValue;
     }
 }
@@ -1423,6 +1438,30 @@ static uint32_t narrow_tile_wt(uint32_t M, uint32_t nt) {
     const size_t cus = (size_t)device_cu_count();
     if ((size_t)((M + 127) / 128) * nt >= cus) return 4u;
     return (size_t)((M + 63) / 64) * nt * 2 > cus ? 2u : 1u;
+}
+
+// 17 to 32 rows whose 16-column tiles fill the CUs unevenly: the 128-column tiles with K in
+// parts, given their workspace, are faster (M = 32, 9728 x 9728 26.9 against 29.0 us, M = 24,
+// 14336 x 2560 13.7 / 14.6).
+static bool skinny_without_split(uint32_t M, uint32_t N, uint32_t K) {
+    const size_t per16 = 16 * (size_t)device_cu_count();   // columns of one 16-column tile per CU
+    return M > 16 && ((K >= 9216 && N > 2 * per16 && 6 * (size_t)((N + GW_N - 1) / GW_N) < (size_t)device_cu_count()) ||
+                      (K > 2048 && K <= 2560 && N > 3 * per16 && 2 * N <= 7 * per16));
+}
+
+// Up to 32 rows, but for shapes that leave its waves without work: one half block of K (K = 64,
+// 8192 columns, M = 8: 3.3 us on the 128-column tiles, 3.7 here), and past 16 rows a few blocks on
+// a few column tiles per CU or very many (M = 32, us, 128-column tiles against this kernel:
+// 12288 x 128 4.3 / 4.8, 16384 x 512 5.9 / 7.1, x 1024 8.1 / 8.9, 65536 x 128 8.3 / 9.7).
+bool w4g_gemm_skinny(uint32_t M, uint32_t N, uint32_t K) {
+    if (M > 32) return false;
+    const size_t per16 = 16 * (size_t)device_cu_count();
+    if (M > kW4gGemvMaxM && K <= 64 && (M > 16 || N <= 5 * per16)) return false;
+    if (M <= 16) return true;
+    if (K <= 256 && N > 2 * per16 && N <= 5 * per16) return false;
+    if (K <= 128 && N > 14 * per16) return false;
+    if (K <= 1024 && N > 3 * per16 && N <= 4 * per16) return false;
+    return !skinny_without_split(M, N, K);
 }
 
 hipError_t launch_w4g_gemm(const __half* a, uint32_t lda, const uint8_t* wq, const __half* ws,
@@ -1445,16 +1484,17 @@ hipError_t launch_w4g_gemm(const __half* a, uint32_t lda, const uint8_t* wq, con
                            nt, K / GB_K, nullptr, R);
         return hipGetLastError();
     }
-    if (w4g_gemm_skinny(M)) return launch_skinny(a, lda, wq, ws, y, ldy, M, N, K, st, epi);
+    const uint32_t parts = w4g_gemm_split_parts(M, N, K);
+    const size_t need = (size_t)parts * M * N * sizeof(float);
+    const bool split = parts > 1 && epi.split_ws && epi.split_ws_bytes >= need;
+    if (w4g_gemm_skinny(M, N, K) || (M <= 32 && skinny_without_split(M, N, K) && !split))
+        return launch_skinny(a, lda, wq, ws, y, ldy, M, N, K, st, epi);
     if (epi.swiglu) {
         const hipError_t te = silu_table_ready(st);
         if (te != hipSuccess) return te;
     }
     const uint32_t mt = (M + GB_M - 1) / GB_M, nt = (N + GB_N - 1) / GB_N, steps = K / GB_K;
     const uint32_t ntw = (N + GW_N - 1) / GW_N;
-    const uint32_t parts = w4g_gemm_split_parts(M, N, K);
-    const size_t need = (size_t)parts * M * N * sizeof(float);
-    const bool split = parts > 1 && epi.split_ws && epi.split_ws_bytes >= need;
     const uint32_t per = split ? (steps + parts - 1) / parts : steps;
     // Both tile shapes give the same bits. The wide one when its grid fills two rounds of
     // two workgroups per CU (measured at M = 2048: gate/up N = 19456 256 vs 263 us; with
@@ -1520,7 +1560,7 @@ hipError_t launch_w4g_gemm(const __half* a, uint32_t lda, const uint8_t* wq, con
 // M = 128, N = 2560, K = 9728 58.2 -> 24.6 us);
 // otherwise two parts of 16+ steps on the 128 x 128 kernel.
 uint32_t w4g_gemm_split_parts(uint32_t M, uint32_t N, uint32_t K) {
-    if (w4g_gemm_skinny(M)) return 1u;   // that kernel splits K inside its workgroups
+    if (w4g_gemm_skinny(M, N, K)) return 1u;   // that kernel splits K inside its workgroups
     const size_t mt = (M + GB_M - 1) / GB_M, cus = (size_t)device_cu_count();
     if (mt * ((N + GB_N - 1) / GB_N) >= 2 * cus) return 1u;
     if (K / GB_K >= 48 && 3 * mt * ((N + GW_N - 1) / GW_N) <= 2 * cus) return 3u;

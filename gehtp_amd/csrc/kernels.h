@@ -58,23 +58,25 @@ struct W4gEpilogue {
 // y[m*ldy + n] = f16( sum_k x[m*ldx + k] * fp16(q[n,k] * s[n, k/64]) ), m < M, n < N,
 // each dequantized weight rounded to fp16 as the reference does, fp32 accumulation
 // (N = weight rows; with swiglu the output has N/2 columns).
+// launch_w4g_gemv: M <= kW4gGemvMaxM, by the GEMV or by the few-row GEMM, whichever is the
+// faster one for the shape; with `gemv_only` by the GEMV.
 hipError_t launch_w4g_gemv(const __half* x, uint32_t ldx, const uint8_t* wq, const __half* ws,
                            __half* y, uint32_t ldy, uint32_t M, uint32_t N, uint32_t K,
-                           hipStream_t st, const W4gEpilogue& epi = W4gEpilogue());
+                           hipStream_t st, const W4gEpilogue& epi = W4gEpilogue(), bool gemv_only = false);
 hipError_t launch_w4g_gemm(const __half* a, uint32_t lda, const uint8_t* wq, const __half* ws,
                            __half* y, uint32_t ldy, uint32_t M, uint32_t N, uint32_t K,
                            hipStream_t st, const W4gEpilogue& epi = W4gEpilogue());
+// Whether launch_w4g_gemm runs w4g_skinny_kernel (up to 32 rows, K split inside its
+// workgroups) for a call without the RoPE epilogue.
+bool w4g_gemm_skinny(uint32_t M, uint32_t N, uint32_t K);
 // K parts the GEMM uses for (M, N, K) when given a workspace, and the workspace bytes
 // (0 when it runs unsplit).
-// M <= 32 rows run w4g_skinny_kernel (K split inside its workgroups) unless the call
-// carries the RoPE epilogue.
-inline bool w4g_gemm_skinny(uint32_t M) { return M <= 32; }
 uint32_t w4g_gemm_split_parts(uint32_t M, uint32_t N, uint32_t K);
 size_t w4g_gemm_split_bytes(uint32_t M, uint32_t N, uint32_t K);
 // w[n*K + k] = fp16(q * s) (bit-exact dequant; used by tests and the fp16 fallback).
 hipError_t launch_w4g_dequant(const uint8_t* wq, const __half* ws, __half* w,
                               uint32_t N, uint32_t K, hipStream_t st);
-// Largest M the GEMV handles; larger M goes to the MFMA GEMM.
+// Largest M the GEMV handles; larger M goes to the MFMA GEMMs.
 constexpr uint32_t kW4gGemvMaxM = 4;
 // True when launch_w4g_gemv runs the GEMV itself for (M, K) (otherwise it hands the
 // call to the GEMM, which cannot take an RMSNorm prologue).

@@ -26,14 +26,16 @@ extern "C" {
 #define GEHTP_E2BIG (-7)   /* request larger than a fixed-size scratch */
 
 /* y[M, ldy] = x[M, ldx] . dequant(W)^T, W4G int4 group-64 (OP_MATMUL_W4G_F16):
- * M <= 2 runs the GEMV, larger M an MFMA GEMM (its few-row form up to 32). Mirrors exec_matmul_f16's scalar
+ * M <= 2 runs the GEMV, 3 and 4 rows it or the MFMA GEMM's few-row form (by the shape),
+ * larger M an MFMA GEMM (its few-row form up to 32). A row's bits do not depend on M from
+ * 33 rows on in calls without a workspace; below, the kernel, and with it the order of the
+ * fp32 sums, changes with M. Mirrors exec_matmul_f16's scalar
  * arithmetic (oplist_exec.c:1802-1811) on dequant(W) = fp16(q*s) with fp32
  * accumulation (summation order differs).
  * K % 64 == 0, ldx % 8 == 0, x and wq 16-byte aligned. */
 int gehtp_w4g_matmul(const void* x, uint32_t ldx, const void* wq, const void* ws, void* y,
                      uint32_t ldy, uint32_t M, uint32_t N, uint32_t K, void* stream);
-/* Force one side of that choice (for measurement): GEMV needs M <= 4 (3 and 4 rows run the
- * GEMM of few rows either way). */
+/* Force one implementation (for measurement): GEMV needs M <= 4. */
 int gehtp_w4g_gemv(const void* x, uint32_t ldx, const void* wq, const void* ws, void* y,
                    uint32_t ldy, uint32_t M, uint32_t N, uint32_t K, void* stream);
 int gehtp_w4g_gemm(const void* x, uint32_t ldx, const void* wq, const void* ws, void* y,

@@ -964,7 +964,12 @@ def test_matmul_f16_gemv_special_values(lib, torch_dev, M, K, N):
 
 
 @pytest.mark.parametrize("M,N,K,mode,norm", [
-    (20, 32784, 320, 0, False), (5, 33000, 192, 1, False), (2, 65552, 128, 0, True)])   # 3 column tiles where 2 would do
+    (8, 20480, 64, 0, False), (8, 20496, 64, 1, False),                              # 128-column tiles / few-row kernel, K = 64
+    (32, 8208, 256, 0, False), (17, 16384, 1024, 1, False), (17, 57360, 128, 0, False),   # 128-column tiles past 16 rows
+    (24, 14336, 2560, 0, False), (32, 8448, 9216, 0, False),                         # their K parts, with a workspace
+    (20, 32784, 320, 0, False), (5, 33000, 192, 1, False), (2, 65552, 128, 0, True),   # 3 column tiles where 2 would do
+    (3, 512, 4096, 0, False), (4, 1000, 8192, 0, False), (3, 512, 8192, 1, False), (3, 9216, 8192, 0, False),   # GEMV
+    (2, 64, 8192, 0, True), (2, 200, 9728, 1, True)])
 def test_w4g_few_rows_forms(lib, oracle, torch_dev, M, N, K, mode, norm):
     """Up to 32 rows where the rules change kernels on 256 CUs: the GEMV, the few-row GEMM (by
     its column tiles per workgroup) and the 128-column tiles, with and without their K parts.
