@@ -811,15 +811,22 @@ hipError_t launch_rmsnorm2(const __half* x, const __half* g, const __half* b, __
 hipError_t launch_softmax(const __half* x, __half* y, uint32_t rows, uint32_t n, hipStream_t st) {
     if (!rows || !n) return hipSuccess;
     const int vector_form = (n % 32 == 0 && (size_t)rows * n >= 32) ? 1 : 0;
-    // A row per wave up to 2048 columns (longer rows would hold over 32 values per lane);
-    // rows spread one to a workgroup while that leaves no CU with more than 4 waves.
+    // A row per wave up to 2048 columns (longer rows would hold over 32 values per lane), rows
+    // one to a workgroup while that leaves no CU with more than 4 waves (6 past 512 columns).
+    // Values per lane in steps of 4 past 512 columns: a lane takes every exponential it holds, so
+    // 16 for a row of 513 cost more than the workgroup per row did (64 rows of 513 x 2 bytes:
+    // 3.3 us with that, 3.8 with 16 values, 3.3 with 12; 64 of 1025: 4.1 / 4.8 / 4.2).
     if (n <= 2048) {
-        const uint32_t wv = rows <= 4u * (uint32_t)device_cu_count() ? 1u : 4u;
+        const uint32_t wv = rows <= (n <= 512 ? 4u : 6u) * (uint32_t)device_cu_count() ? 1u : 4u;
         const auto kern = n < 64      ? softmax_wave_kernel<1, 1>
                           : n <= 128  ? softmax_wave_kernel<2, 1>
                           : n <= 256  ? softmax_wave_kernel<4, 1>
                           : n <= 512  ? softmax_wave_kernel<8, 1>
+                          : n <= 768  ? softmax_wave_kernel<4, 3>
                           : n <= 1024 ? softmax_wave_kernel<8, 2>
+                          : n <= 1280 ? softmax_wave_kernel<4, 5>
+                          : n <= 1536 ? softmax_wave_kernel<8, 3>
+                          : n <= 1792 ? softmax_wave_kernel<4, 7>
                                       : softmax_wave_kernel<8, 4>;
         hipLaunchKernelGGL(kern, dim3((rows + wv - 1) / wv), dim3(64 * wv), 0, st, x, y, rows, n, vector_form);
         return hipGetLastError();

@@ -908,10 +908,11 @@ def test_w4g_few_rows_norm(lib, oracle, torch_dev, M, N, K, mode, use_res):
 
 
 @pytest.mark.parametrize("rows,n", [(1, 1), (9, 2), (5, 63), (3, 64), (70, 32), (6, 129), (3, 255), (2, 257), (7, 511), (1030, 512), (4, 513), (9, 1024), (1100, 1001),
-                                    (6, 2048), (5, 2049), (5, 7)])
+                                    (6, 2048), (5, 2049), (5, 7), (9, 768), (5, 769), (2050, 1025), (3, 1280), (3, 1281),
+                                    (4, 1536), (5, 1537), (2, 1792), (3, 1793)])
 def test_softmax_row_per_wave(lib, torch_dev, rows, n):
-    """The row-per-wave softmax (n <= 2048: chunks of 1, 2, 4 or 8 values, 1, 2 or 4 per lane, one
-    or four rows per workgroup) and the longer rows beside it, at row lengths off every alignment, from a
+    """The row-per-wave softmax (n <= 2048: chunks of 1, 2, 4 or 8 values, 1, 2, 3, 4, 5 or 7 per lane,
+    one or four rows per workgroup) and the longer rows beside it, at row lengths off every alignment, from a
     pointer 2 bytes off, in place, with -inf entries (a masked row's shape). Against float64:
     one fp16 rounding of the exponential and one of the quotient (2^-10 together), the fp32
     exponential and sum (n 2^-24) besides."""
@@ -996,3 +997,32 @@ def test_w4g_few_rows_forms(lib, oracle, torch_dev, M, N, K, mode, norm):
         got = from_dev(y)
         assert (got[M] == 7).all()
         assert_close(got[:M], ref, what=f"{M}x{N}x{K} mode={mode} norm={norm} work={work is not None}")
+
+
+@pytest.mark.parametrize("n", [61, 64, 128, 256, 500, 512, 700, 1000, 1024, 1100, 1280, 1536, 1700, 1800, 2048, 2100, 2112])
+def test_softmax_special_rows(lib, torch_dev, n):
+    """Rows with a +inf, a NaN, all -inf, and all at the lowest finite value, between ordinary
+    rows: the vector form (n a multiple of 32) scales by 0 when the sum is no positive number,
+    the other divides by it, and the ordinary rows keep their bits. Rows per wave and (past
+    2048 columns) per workgroup alike."""
+    import torch
+    g = torch.Generator(device=torch_dev).manual_seed(n)
+    x = (torch.randn((9, n), device=torch_dev, generator=g) * 3).half()
+
+    def run(x):
+        y = torch.empty_like(x)
+        assert lib.gehtp_softmax(ptr(x), ptr(y), x.shape[0], n, stream_ptr()) == 0
+        _sync()
+        return y
+
+    clean, hot = run(x), x.clone()
+    hot[1, n - 1], hot[3, n // 2], hot[5], hot[7] = float("inf"), float("nan"), float("-inf"), -65504
+    got = run(hot)
+    assert torch.equal(got[::2].view(torch.int16), clean[::2].view(torch.int16))
+    nan = torch.zeros((9, n), dtype=torch.bool, device=torch_dev)
+    nan[1, n - 1] = nan[3, n // 2] = nan[5] = True
+    if n % 32:
+        nan[1] = nan[3] = True
+    assert torch.equal(torch.isnan(got), nan)
+    assert (got[[1, 3]][~nan[[1, 3]]] == 0).all()
+    assert ((got[7].double() - 1 / n).abs() <= 2 ** -10 / n + 2 ** -24).all()
