@@ -1033,41 +1033,56 @@ __global__ __launch_bounds__(256) void merge_oproj_kernel(MergeOprojArgs M) {
 }
 
 // The tile of a prefill: queries per tile (32 wph), parts over the keys, and its measured
-// cost in units of 0.1 us: `base` for a workgroup plus `step` per key stage of a part (one
-// workgroup per CU; S 128..2048, 8/16/32 heads, both masks, fitted within ~5 %).
+// cost in units of 10 ns: `launch` for the call, `base` for a workgroup plus `step` per key
+// stage of a part, one workgroup per CU (152 KB of LDS). S 1..4096, 1..128 heads, both masks:
+// within 10 % of the measured time in nine cases of ten, 20 % at worst.
 //
-// One round of workgroups takes its heaviest member's time. More workgroups than CUs:
-// without a mask all are alike and every begun round costs one; with it, heavy first,
-// the mean load times 1.1 (the tail) once that is larger. Measured, us (32-query x 2
-// parts / 64 x 2 / 128 x 2 / 32 x 4 / 64 x 4), the rule's choice marked:
+// Up to one workgroup per CU the heaviest sets the time. More: without a mask all are alike
+// and every begun round costs one. With it they are handed out heavy first, so the time is at
+// least the mean load (times 1.15 for the tail) and what the first and the last CU to get a
+// second workgroup run. Measured, us (32-query x 2 parts / 64 x 2 / 128 x 2 / 32 x 4 / 64 x 4),
+// the rule's choice marked:
+//   S  200 x 40 heads causal   12.1 / *9.5 / 10.2 / 15.6 / 10.4
 //   S  256 x 16 heads causal   *8.2 / 8.9 / 10.6 / 8.2 / 9.7
 //   S  512 x 32 heads causal   18.3 / *13.4 / 15.0 / 19.2 / 13.4
+//   S  768 x 24 heads causal   26.9 / *17.2 / 18.6 / 27.8 / 19.0
 //   S  768 x 32 heads          44.8 / 30.3 / *18.9 / 38.5 / 30.5
 //   S 1024 x  8 heads causal   19.7 / 19.4 / 21.0 / *16.3 / 17.8
 //   S 1024 x 16 heads causal   25.9 / 20.1 / 22.0 / 24.2 / *18.6
 //   S 1536 x 16 heads          78.3 / 50.4 / *29.6 / 62.3 / 46.4
 //   S 2048 x 32 heads causal   158 / 77 / *52.8 / 134 / 80
-// (The largest tile that still fills the CUs, which stood here before, took 31.8 us for
-// the third line, 52.8 for the sixth: two rounds of 64-query tiles.)
 //
 // Four parts only past 8 stages (S > 512): below, the outputs are the same bits whatever
 // the tile (two parts split the stages of an enclosing tile where it does), and four
 // parts gain nothing up to S = 384 and ~1 us at 512.
 struct AttnTile {
-    uint32_t wph, np, base, step;
+    uint32_t wph, np;
+    int64_t launch, base, step;
 };
-constexpr AttnTile kAttnTiles[5] = {{4, 2, 59, 19}, {2, 2, 47, 18}, {1, 2, 38, 20}, {2, 4, 60, 30}, {1, 4, 49, 28}};
+constexpr AttnTile kAttnTiles[5] = {
+    {4, 2, -160, 770, 200}, {2, 2, 70, 510, 170}, {1, 2, 150, 350, 180}, {2, 4, -30, 650, 290}, {1, 4, 70, 380, 290}};
 
 AttnTile attn_prefill_form(uint32_t S, uint32_t H, bool causal) {
-    const uint64_t cus = (uint64_t)device_cu_count(), ns = ((uint64_t)S + KT - 1) / KT;
+    const int64_t cus = device_cu_count(), ns = ((int64_t)S + KT - 1) / KT;
     AttnTile best = kAttnTiles[0];
-    uint64_t best_cost = UINT64_MAX;
+    int64_t best_cost = INT64_MAX;
     for (const AttnTile& f : kAttnTiles) {
         if (f.np == 4 && ns <= 8) continue;
-        const uint64_t qt = 32 * f.wph, wgs = (uint64_t)H * ((S + qt - 1) / qt), steps = (ns + f.np - 1) / f.np;
-        uint64_t cost = f.base + f.step * steps;
-        if (!causal) cost *= (wgs + cus - 1) / cus;
-        else if (wgs > cus) cost = std::max(cost, (2 * f.base + f.step * (steps + 1)) * wgs * 11 / (20 * cus));
+        const int64_t qt = 32 * f.wph, nqt = ((int64_t)S + qt - 1) / qt, wgs = H * nqt;
+        auto wg = [&](int64_t g) {   // cost of a workgroup of the g-th tile of a head, heavy first
+            const int64_t kend = causal ? std::min<int64_t>(S, (nqt - g) * qt) : S;
+            return f.base + f.step * (((kend + KT - 1) / KT + f.np - 1) / f.np);
+        };
+        int64_t cost = wg(0);
+        if (wgs > cus && !causal) {
+            cost *= (wgs + cus - 1) / cus;
+        } else if (wgs > cus) {
+            const int64_t last = std::min(wgs - cus, cus) - 1;   // second workgroups: numbers cus .. cus + last
+            cost = std::max(cost, (wg(0) + wg(nqt - 1)) * wgs * 23 / (40 * cus));
+            cost = std::max(cost, wg((cus - 1) / H) + wg(cus / H));
+            cost = std::max(cost, wg((cus - 1 - last) / H) + wg((cus + last) / H));
+        }
+        cost += f.launch;
         if (cost < best_cost) {
             best_cost = cost;
             best = f;

@@ -375,9 +375,8 @@ def test_attn_prefill_wide_ragged(lib, oracle, torch_dev, ramp):
 
 @pytest.mark.parametrize("causal", [False, True])
 def test_attn_prefill_tile_sizes(lib, oracle, torch_dev, causal):
-    """The prefill runs 128-query tiles when heads x tiles cover the CUs (256 on MI355X),
-    else 64-query tiles when those do (config 3: 16 heads x 16 tiles), else 32-query
-    tiles. At S = 512, 64 heads take the 128-query tiles, their first 32 heads (over the
+    """The prefill runs 128-, 64- or 32-query tiles by their modelled cost (past 512 tokens
+    also with four key parts). On 256 CUs at S = 512, 64 heads take the 128-query tiles, their first 32 heads (over the
     first 4 KV heads, the same grouping) the 64-query ones and their first 16 the
     32-query ones. Every query sums the same key stages in the same order each time
     (with the mask too: a tile's two halves split its stages where the enclosing larger
@@ -406,13 +405,14 @@ def test_attn_prefill_tile_sizes(lib, oracle, torch_dev, causal):
 
 
 @pytest.mark.parametrize("S,H,causal", [(513, 8, True), (600, 16, True), (577, 8, False), (700, 16, False), (641, 48, True),
-                                        (769, 32, False)])
+                                        (769, 32, False), (700, 16, True), (1001, 16, True), (768, 24, True)])
 def test_attn_prefill_four_parts(lib, oracle, torch_dev, S, H, causal):
     """Past 512 tokens, grids of up to one workgroup per CU split a tile's key stages over
-    four parts (32-query tiles at 8 heads, 64-query at 16; 9 stages of 513..576 tokens leave
-    the last part empty, and one key in the last stage at 513, 577); larger grids (48 heads,
-    32 without a mask) take two parts. Keys grow along S, so that late stages move the
-    reference max and the parts' maxima differ."""
+    four parts (32-query tiles at 8 heads; 64-query ones at 16 heads and 700 or 1001 tokens,
+    causal with a partial last key stage and query tile; 9 stages of 513..576 tokens leave the
+    last part empty, and one key in the last stage at 513, 577); larger grids (48 heads, 24
+    at 768 tokens, 32 without a mask) and 600 tokens of 16 heads take two parts. Keys grow
+    along S, so that late stages move the reference max and the parts' maxima differ."""
     import torch
     rng = np.random.default_rng(S)
     KVH, hd = 8, 128
