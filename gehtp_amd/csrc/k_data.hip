@@ -67,8 +67,8 @@ __global__ void crouton_decode_kernel(const uint32_t* __restrict__ surf, uint16_
 // in one word, odd ones in the other; A's columns are staged in that order), and the sums,
 // all multiples of 16, are shifted down exactly.
 // Workgroup tile 32 RT x 32 NT, its K steps (64 = two 32-column blocks of the surface)
-// split over 8 waves in contiguous ranges: at these sizes (M = 256, K = N = 2560: 160 tiles
-// of 64 x 64) a serial K loop is latency. Each wave stages its own A block in LDS
+// split over WV = 8 waves in contiguous ranges (one wave for short K on large grids): at
+// M = 256, K = N = 2560 (160 tiles of 64 x 64) a serial K loop is latency. Each wave stages its own A block in LDS
 // (256 RT-byte runs of the surface in, byte planes out), so its loop needs no barrier; W
 // goes from memory to the B operand. The waves' sums meet in LDS. int32 holds the tile's
 // whole sums up to 8064 columns (8064 * 32896 * 8 < 2^31); longer K runs in such chunks with
@@ -77,7 +77,6 @@ __global__ void crouton_decode_kernel(const uint32_t* __restrict__ surf, uint16_
 // CU's cycles (the byte planes: 24 instructions per 16 u16 pairs), LDS 41 %, L1 55 %, MFMA
 // 24 %. 256 x 2560 x 2560: 134.9 -> 12.5 us per call (the 64 x 64 v_dot2 tiles it replaces, one wave
 // row per 16 columns and a barrier per 32 columns, against this).
-constexpr uint32_t WA_WV = 8;
 constexpr uint32_t kWaChunk = 126;   // K steps of an int32 chunk: 8064 columns
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
@@ -90,18 +89,18 @@ __device__ __forceinline__ uint32_t w4a16_out(T s) {
     return y < 0 ? 0u : y > 65535 ? 65535u : (uint32_t)y;
 }
 
-template <int RT, int NT, int MINW>
-__global__ __launch_bounds__(64 * WA_WV, MINW) void w4a16_gemm_kernel(const uint16_t* __restrict__ act,
-                                                                      const uint8_t* __restrict__ w,
-                                                                      uint16_t* __restrict__ out, uint32_t M,
-                                                                      uint32_t K, uint32_t N) {
+template <int RT, int NT, int MINW, uint32_t WV>
+__global__ __launch_bounds__(64 * WV, MINW) void w4a16_gemm_kernel(const uint16_t* __restrict__ act,
+                                                                   const uint8_t* __restrict__ w,
+                                                                   uint16_t* __restrict__ out, uint32_t M,
+                                                                   uint32_t K, uint32_t N) {
     // A staged plane: rows of 64 bytes at a stride of 80 (operand reads of 16 rows and
     // stores of every second row then spread over all banks), 128 bytes between row tiles.
     constexpr uint32_t RS = 80, TS = 32 * RS + 128, PLANE = RT * TS, NU = 2 * RT;
     constexpr uint32_t CS = 32 * RT + 4, TILE = 32 * CS;   // a wave's sums of one n tile: [column][row], padded
-    constexpr uint32_t NQ = RT * 512 / (64 * WA_WV);       // surface words per thread and n tile
+    constexpr uint32_t NQ = RT * 512 / (64 * WV);          // surface words per thread and n tile
     constexpr uint32_t WLDS = 2 * PLANE > TILE * 4 ? 2 * PLANE : TILE * 4;
-    __shared__ __align__(16) uint8_t lds[WA_WV * WLDS];
+    __shared__ __align__(16) uint8_t lds[WV * WLDS];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5, l32 = lane & 31;
     const uint32_t n_m32 = M >> 5, n_kt = K >> 5, nsteps = (n_kt + 1) / 2;
     const uint32_t nt = (N / 32 + NT - 1) / NT, g0 = (blockIdx.x / nt) * RT, n0 = (blockIdx.x % nt) * (32 * NT);
@@ -141,7 +140,7 @@ __global__ __launch_bounds__(64 * WA_WV, MINW) void w4a16_gemm_kernel(const uint
         for (uint32_t e = 0; e < 2 * NQ; ++e) tot[j][e >> 1][e & 1] = 0;
 
     for (uint32_t c0 = 0; c0 < nsteps; c0 += kWaChunk) {
-        const uint32_t cn = min(kWaChunk, nsteps - c0), per = (cn + WA_WV - 1) / WA_WV;
+        const uint32_t cn = min(kWaChunk, nsteps - c0), per = (cn + WV - 1) / WV;
         const uint32_t s0 = c0 + min(wave * per, cn), s1 = c0 + min((wave + 1) * per, cn);
         i32x16 acc[NT][2][RT];   // [n tile][plane][row tile]
         int wsum[NT];
@@ -215,7 +214,7 @@ __global__ __launch_bounds__(64 * WA_WV, MINW) void w4a16_gemm_kernel(const uint
             __builtin_amdgcn_wave_barrier();
         }
         // Sums over the waves, one n tile at a time: [wave][column][row]. Thread t holds
-        // surface words (row pair, column) = t, t + 512.
+        // surface words (row pair, column) = t, t + 64 WV, ...
         int* red = reinterpret_cast<int*>(lds);
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
@@ -232,10 +231,10 @@ __global__ __launch_bounds__(64 * WA_WV, MINW) void w4a16_gemm_kernel(const uint
             __syncthreads();
 #pragma unroll
             for (uint32_t q = 0; q < NQ; ++q) {
-                const uint32_t idx = tid + 512 * q, col = idx & 31, pr = idx >> 5;
+                const uint32_t idx = tid + 64 * WV * q, col = idx & 31, pr = idx >> 5;
                 int sum[2] = {0, 0};
 #pragma unroll
-                for (uint32_t v = 0; v < WA_WV; ++v) {
+                for (uint32_t v = 0; v < WV; ++v) {
                     const int2 x = *reinterpret_cast<const int2*>(&red[v * TILE + col * CS + 2 * pr]);
                     sum[0] += x.x;
                     sum[1] += x.y;
@@ -246,13 +245,13 @@ __global__ __launch_bounds__(64 * WA_WV, MINW) void w4a16_gemm_kernel(const uint
         }
         __syncthreads();
 #pragma unroll
-        for (int j = 0; j < NT; ++j) red[(j * WA_WV + wave) * 64 + lane] = wsum[j] >> 4;   // this lane's k half of column l32
+        for (int j = 0; j < NT; ++j) red[(j * WV + wave) * 64 + lane] = wsum[j] >> 4;   // this lane's k half of column l32
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
             int ws = 0;
 #pragma unroll
-            for (uint32_t v = 0; v < 2 * WA_WV; ++v) ws += red[j * WA_WV * 64 + v * 32 + (tid & 31)];
+            for (uint32_t v = 0; v < 2 * WV; ++v) ws += red[j * WV * 64 + v * 32 + (tid & 31)];
 #pragma unroll
             for (uint32_t e = 0; e < 2 * NQ; ++e) tot[j][e >> 1][e & 1] += (int64_t)ws * 128;
         }
@@ -265,7 +264,7 @@ __global__ __launch_bounds__(64 * WA_WV, MINW) void w4a16_gemm_kernel(const uint
     for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (uint32_t q = 0; q < NQ; ++q) {
-            const uint32_t idx = tid + 512 * q, col = idx & 31, m = g0 * 32 + 2 * (idx >> 5), kt = (n0 >> 5) + j;
+            const uint32_t idx = tid + 64 * WV * q, col = idx & 31, m = g0 * 32 + 2 * (idx >> 5), kt = (n0 >> 5) + j;
             if (m >= M || kt >= on_kt) continue;
             uint32_t v[2];
 #pragma unroll
@@ -454,12 +453,16 @@ hipError_t launch_matmul_w4a16(const uint16_t* act, const uint8_t* w, uint16_t* 
     const double r11 = rounds(grid(1, 1));
     const double t11 = 8.3 * std::floor(r11 / 2) + 5.8 * std::fmod(r11, 2.0);
     const double t12 = 8.2 * rounds(grid(1, 2)), t22 = 12.0 * rounds(grid(2, 2));
-    auto go = [&](auto kern, uint32_t rt, uint32_t nt) {
-        hipLaunchKernelGGL(kern, dim3((uint32_t)grid(rt, nt)), dim3(64 * WA_WV), 0, st, act, w, out, M, K, N);
+    auto go = [&](auto kern, uint32_t rt, uint32_t nt, uint32_t wv) {
+        hipLaunchKernelGGL(kern, dim3((uint32_t)grid(rt, nt)), dim3(64 * wv), 0, st, act, w, out, M, K, N);
     };
-    if (t22 < t11 && t22 < t12) go(w4a16_gemm_kernel<2, 2, 2>, 2, 2);
-    else if (t12 < t11) go(w4a16_gemm_kernel<1, 2, 2>, 1, 2);
-    else go(w4a16_gemm_kernel<1, 1, 4>, 1, 1);
+    // One or two K steps leave most of 8 waves without work, so large grids run one wave per tile
+    // (M x N x K, us, 8 waves / one): 2048 x 2560 x 32 26.5 / 12.7, x 128 26.6 / 13.8, 1024 x 1024
+    // x 128 6.7 / 7.1.
+    if (K <= 128 && grid(1, 2) > 2 * cus) go(w4a16_gemm_kernel<1, 2, 1, 1>, 1, 2, 1);
+    else if (t22 < t11 && t22 < t12) go(w4a16_gemm_kernel<2, 2, 2, 8>, 2, 2, 8);
+    else if (t12 < t11) go(w4a16_gemm_kernel<1, 2, 2, 8>, 1, 2, 8);
+    else go(w4a16_gemm_kernel<1, 1, 4, 8>, 1, 1, 8);
     return hipGetLastError();
 }
 

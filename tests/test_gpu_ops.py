@@ -256,12 +256,14 @@ def test_engine_data_ops(engine, oracle):
 
 
 @pytest.mark.parametrize("M,K,N", [(32, 32, 96), (32, 96, 1056), (64, 8064, 64), (64, 8096, 32), (96, 544, 4064),
-                                   (256, 576, 2592), (1024, 160, 544)])
+                                   (256, 576, 2592), (1024, 160, 544),
+                                   (1056, 32, 1056), (1056, 96, 1056), (2048, 128, 544)])
 def test_matmul_w4a16_tiles(lib, oracle, torch_dev, M, K, N):
     """Opcode 1's tile shapes and remainders on 256 CUs: 32 x 32, 32 x 64 and 64 x 64 tiles,
     an odd row or column tile at the edge, an odd number of 32-column blocks (the last K
-    step half empty), fewer K steps than waves, and K on both sides of the longest int32
-    chunk with every product at its largest. Whole numbers: bit for bit."""
+    step half empty), fewer K steps than waves, one-wave tiles for K up to 128 on large grids,
+    and K on both sides of the longest int32 chunk with every product at its largest. Whole
+    numbers: bit for bit."""
     import torch
     rng = np.random.default_rng(M + K + N)
     A = rng.integers(0, 65536, size=(M, K), dtype=np.uint16)
