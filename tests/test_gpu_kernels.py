@@ -743,14 +743,15 @@ def test_qk_rope_kv(lib, oracle, torch_dev, n_tok, H, KVH):
     assert rk.max() <= 1 and (rk == 0).mean() > 0.999
 
 
-@pytest.mark.parametrize("H,KVH,pos0", [(32, 8, 100), (16, 8, 63), (8, 8, 0), (16, 2, 130)])
+@pytest.mark.parametrize("H,KVH,pos0", [(32, 8, 100), (16, 8, 63), (8, 8, 0), (16, 2, 130),
+                                        (16, 8, 4094), (32, 8, 4157), (8, 2, 8190)])   # second and third merge round
 def test_attn_decode_qkv_matches_unfused(lib, oracle, torch_dev, H, KVH, pos0):
     """OP_ATTN_DECODE_QKV_F16 = OP_QK_ROPE_KV_F16 (one token) + OP_ATTN_DECODE_F16 at the
     advanced counter: same ring bytes, same counter and bit-identical outputs over three
     consecutive steps, and the attention output within the parity bar of the oracle."""
     import torch
     rng = np.random.default_rng(H * 1000 + KVH * 10 + pos0)
-    hd, nslots = 128, 256
+    hd, nslots = 128, 256 if pos0 < 250 else 12288
     kv_elems = KVH * hd
     state_bytes = nslots * kv_elems * 4
     ring_ref = oracle.KVRing(state_bytes, kv_elems)

@@ -89,7 +89,13 @@ def test_qkv_attn_one_launch_matches_two_kernels(lib, oracle, torch_dev, H, KVH,
 
 @pytest.mark.parametrize("H,KVH,K,nslots,pos0,with_res", [(32, 8, 2560, 4096, 2059, True),
                                                           (16, 8, 1024, 256, 63, False),
-                                                          (8, 8, 2048, 128, 0, True)])
+                                                          (8, 8, 2048, 128, 0, True),
+                                                          # past 64 chunks: the merge's later rounds, handed on to
+                                                          # the o-proj's 16- and 32-lane rows
+                                                          (16, 8, 1024, 4608, 4094, True),
+                                                          (32, 8, 2560, 4608, 4157, True),
+                                                          (8, 8, 2048, 4608, 4480, False),
+                                                          (16, 4, 1024, 8704, 8190, True)])
 def test_qkv_attn_oproj_two_launches_match_separate_calls(lib, torch_dev, H, KVH, K, nslots, pos0, with_res):
     """gehtp_qkv_attn_oproj_decode (the q|k|v GEMV + chunk pass, then the merge pass + the
     o-proj GEMV reading the attention output from the merge workgroups' records) against
