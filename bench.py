@@ -571,7 +571,7 @@ def kernel_configs(args) -> int:
                                           H, KVH, HD_ATTN, scale, 1, sp) == 0
         t_rot = timed(c3p, copies, 5)
         t_res = timed(lambda i: c3p(0), 32, 5)
-        results["c3_attn_prefill"] = {"kernel": "attn_prefill_kernel<true, WPH>", "flops": flops, "copies": copies,
+        results["c3_attn_prefill"] = {"kernel": "attn_prefill_kernel<true, WPH, NP>", "flops": flops, "copies": copies,
                                       "rotated_us": round(t_rot * 1e6, 3),
                                       "rotated_tflops": round(flops / t_rot / 1e12, 1),
                                       "resident_us": round(t_res * 1e6, 3),
@@ -594,7 +594,7 @@ def kernel_configs(args) -> int:
                                           H, KVH, HD_ATTN, scale, 1, sp) == 0
         t_rot = timed(a4b, copies, 10)
         t_res = timed(lambda i: a4b(0), 32, 5)
-        results["attn_prefill_4b"] = {"kernel": "attn_prefill_kernel<true, 4>", "S": S, "H": H, "KVH": KVH,
+        results["attn_prefill_4b"] = {"kernel": "attn_prefill_kernel<true, 4, 2>", "S": S, "H": H, "KVH": KVH,
                                       "flops": flops, "copies": copies, "rotated_us": round(t_rot * 1e6, 3),
                                       "rotated_tflops": round(flops / t_rot / 1e12, 1),
                                       "resident_us": round(t_res * 1e6, 3),

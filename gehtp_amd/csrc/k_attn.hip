@@ -46,8 +46,8 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const _Float16* p) {
 }
 
 // Flash attention forward. A workgroup owns 32 WPH queries of one head (wave w of a
-// part: queries 32w..32w+31); per 64-key stage, K and V are staged row-major in LDS (the next stage's
-// loads are in flight during the compute). Scores are computed transposed,
+// part: queries 32w..32w+31); per 64-key stage, K and V are staged row-major in LDS (the
+// next stage's loads are in flight during the compute). Scores are computed transposed,
 // S^T = K Q^T (MFMA A = K rows, B = Q^T held in registers), so each lane owns one query
 // and its 32 scores of a stage; the online-softmax statistics need one exchange with
 // lane l^32. O^T = V^T P^T: the V^T operand comes from the row-major V tile through the
@@ -65,9 +65,10 @@ __device__ __forceinline__ u32x2 lds_read_tr16(const _Float16* p) {
 //
 // What bounds it: a lone wave per SIMD takes ~1.9 us per stage (32 MFMAs, then ~220
 // vector instructions, little of either overlapped), on top of 4-6 us of launch, first
-// loads and merge. Two parts (2 or 4 waves: one per SIMD at most) double-buffer the
-// stages, 152 KB of LDS, one barrier per stage; four parts give a SIMD two waves at 64
-// queries (3.0 us for their two stages) and half the steps, in the same LDS, one buffer.
+// loads and merge. Two parts double-buffer the stages, 152 KB of LDS, one barrier per
+// stage: at 32 and 64 queries 2 and 4 waves, one per SIMD at most, at 128 eight, two per
+// SIMD. Four parts give a SIMD two waves at 64 queries (3.0 us for their two stages) and
+// half the steps, in the same LDS, one buffer.
 // attn_prefill_form has the rule between the five forms and what each measured.
 constexpr uint32_t KV_HALF = KT * KS + KT * VSR;   // fp16 values of one LDS K + V stage
 

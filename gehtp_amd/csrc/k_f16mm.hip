@@ -263,8 +263,10 @@ __global__ __launch_bounds__(256) void gemv_col_kernel(const __half* __restrict_
 // back to end there (their columns are computed twice, with the same bits). Operands whose
 // stored rows hold fewer than 8 elements go element by element, zero past the edge.
 // Bound: below one round of the CUs the K loop's latency (0.27 us per step of 64 at 64 x 64),
-// above it LDS reads and MFMA (1024 x 4096 x 4096: 49 us, 700 TFLOP/s). 512 x 3072 x 1024:
-// 123.8 -> 11.0 us against 64 x 64 tiles filled by single elements with two barriers per 32.
+// then LDS (512 x 3072 x 1024, 384 tiles of 64 x 64: 73 % of a busy CU's cycles, L1 42 %, MFMA
+// 16 %, VALU 13 %), and on large grids LDS reads and MFMA (1024 x 4096 x 4096: 49 us, 700
+// TFLOP/s). 512 x 3072 x 1024: 123.8 -> 11.0 us against 64 x 64 tiles filled by single elements
+// with two barriers per 32.
 __device__ __forceinline__ uint2 lds_read_tr16(const _Float16* p) {
     const s4_t r = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
         (__attribute__((address_space(3))) s4_t*)(const_cast<_Float16*>(p)));

@@ -703,18 +703,20 @@ __global__ __launch_bounds__(256, 3) void w4g_gemm_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// GEMM of few rows (M <= 32, w4g_gemm_skinny): weights stream once, so a tile is 16 NT columns of all M rows
-// (AR >= M of them staged; with NORM, M <= 4, normalized as they are staged) and K is split over the workgroup's WV waves in contiguous ranges
-// of 128-deep blocks, their sums added in LDS in wave order; no workspace, one launch. On
-// v_mfma_f32_16x16x32_f16 lane l supplies column (A row) l % 16 and, with j = l / 16, the k's
-// 32 j + 8 q + 0..7 of a block for MFMA q, so a lane's 16 bytes are the weight words of four
-// MFMAs. Loading them that way makes four neighbouring lanes touch four rows (the L1 looks
-// up a line per lane); instead 4 lanes take 64 consecutive bytes of a row, A rows go 256
-// bytes at a time, and both pass through the wave's own LDS space (no barrier), A in the
-// dequant's pair order. A block's loads are issued during the block before it.
-// Bound: VALU issue (the exact dequant, 13 per 8 weights, and the staging) and the L1's
-// lookups (39 and 77 % of the cycles at 8 x 19456 x 2560 before the staging), with the
-// tiles on the busiest CU. Four blocks of loads in flight instead of one were slower (most
+// GEMM of few rows (w4g_gemm_skinny: up to 32): weights stream once, so a tile is 16 NT columns
+// of all M rows (AR >= M of them staged; with NORM, M <= 4, normalized as they are staged) and K
+// is split over the workgroup's WV waves in contiguous ranges of 128-deep blocks, their sums
+// added in LDS in wave order; no workspace, one launch. On v_mfma_f32_16x16x32_f16 lane l
+// supplies column (A row) l % 16 and, with j = l / 16, the k's 32 j + 8 q + 0..7 of a block for
+// MFMA q, so a lane's 16 bytes are the weight words of four MFMAs. Loading them that way makes
+// four neighbouring lanes touch four rows (the L1 looks up a line per lane); instead 4 lanes
+// take 64 consecutive bytes of a row, A rows go 256 bytes at a time, and both pass through the
+// wave's own LDS space (no barrier), A in the dequant's pair order. A block's loads are issued
+// during the block before it.
+// Bound: latency, one or two waves per SIMD with one block of loads in flight each. Of a busy
+// CU's cycles at 8 x 19456 x 2560 (NT 5, 4 waves): VALU 36 % (1945 a wave; the exact dequant, 13
+// per 8 weights, and the staging), LDS 27 %, L1 lookups 18 %, MFMA 7 %; at 8 x 2560 x 9728 (NT 1,
+// 8 waves): 39, 44, 31 and 7 %. Four blocks of loads in flight instead of one were slower (most
 // waves run 3-5 blocks, and the surplus loads cost lookups). M = 8, us against the 128-column
 // tiles of 32 or 128 rows it replaces (60 to 152 workgroups): 2560 x 9728 22.6 -> 9.5,
 // 19456 x 2560 26.7 -> 12.5, 6144 x 2560 10.9 -> 5.3, 4096 x 1024 6.8 -> 3.4; M = 24: 23.1 ->
