@@ -714,7 +714,7 @@ __global__ __launch_bounds__(256, 3) void w4g_gemm_kernel(
 // wave's own LDS space (no barrier), A in the dequant's pair order. A block's loads are issued
 // during the block before it.
 // Bound: latency, one or two waves per SIMD with one block of loads in flight each. Of a busy
-// CU's cycles at 8 x 19456 x 2560 (NT 5, 4 waves): VALU 36 % (1945 a wave; the exact dequant, 13
+// CU's cycles at 8 x 19456 x 2560 (NT 5, 4 waves): VALU 35 % (1945 a wave; the exact dequant, 13
 // per 8 weights, and the staging), LDS 27 %, L1 lookups 18 %, MFMA 7 %; at 8 x 2560 x 9728 (NT 1,
 // 8 waves): 39, 44, 31 and 7 %. Four blocks of loads in flight instead of one were slower (most
 // waves run 3-5 blocks, and the surplus loads cost lookups). M = 8, us against the 128-column

@@ -71,7 +71,8 @@ int gehtp_qk_rope_kv(const void* qkv, uint32_t n_tok, uint32_t H, uint32_t KVH,
 /* w[N, K] fp16 = fp16(q * s): the dequant, bit-exact. */
 int gehtp_w4g_dequant(const void* wq, const void* ws, void* w, uint32_t N, uint32_t K, void* stream);
 
-/* OP_MATMUL_F16 / _SPLIT semantics (oplist_exec.c:1709-1813), flags as in the op. */
+/* OP_MATMUL_F16 / _SPLIT semantics (oplist_exec.c:1709-1813), flags as in the op. A window
+ * [n0, n0 + N) has the bits of the whole product of N_full columns. */
 int gehtp_matmul_f16(const void* a, const void* w, void* y, uint32_t M, uint32_t K,
                      uint32_t N_full, uint32_t n0, uint32_t N, uint32_t flags, void* stream);
 
