@@ -206,7 +206,8 @@ __global__ __launch_bounds__(256) void softmax_kernel(const __half* __restrict__
 // Bound: the exponentials (about 20 VALU each) and one memory round trip, so short rows
 // take short chunks (976 rows of 61: 3.4 us with 8-element chunks on 8 lanes). 8192 rows
 // of 512: 12.4 -> 6.4 us (graph-timed; one workgroup per row, two-byte loads in three
-// passes before), 4096 of 256: 5.7 -> 3.4.
+// passes before), 4096 of 256: 5.7 -> 3.4; 2048 columns (32 values per lane) 64 rows 5.5 ->
+// 4.4, 4096 rows 17.4 -> 10.9.
 template <int E, int C>
 __global__ __launch_bounds__(256) void softmax_wave_kernel(const __half* __restrict__ x,
                                                            __half* __restrict__ y, uint32_t rows,

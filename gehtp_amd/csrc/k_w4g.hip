@@ -1388,7 +1388,8 @@ hipError_t launch_w4g_gemv(const __half* x, uint32_t ldx, const uint8_t* wq, con
         hipError_t e = hipSuccess;
         if (gemv_rw_launch(GemvRwArgs{x, wq, ws, y, N, K, epi.gamma, epi.res, epi.swiglu ? 1 : 0}, st, &e)) return e;
     }
-    if (!gemv_only && !gemv_rows(M, N, K, epi.gamma != nullptr, epi.swiglu)) return launch_skinny(x, ldx, wq, ws, y, ldy, M, N, K, st, epi);
+    if ((!gemv_only || epi.gamma) && !gemv_rows(M, N, K, epi.gamma != nullptr, epi.swiglu))
+        return launch_skinny(x, ldx, wq, ws, y, ldy, M, N, K, st, epi);
     // Rows per workgroup: about two workgroups per CU (three when one workgroup holds a
     // single row per pass, as for K = 9728: measured 11 % faster there, slower for the
     // multi-row shapes), partial sums within 32 KiB.
@@ -1423,6 +1424,8 @@ hipError_t launch_w4g_gemv(const __half* x, uint32_t ldx, const uint8_t* wq, con
     switch (M) {
     case 1: return gemv_dispatch<1>(g3, b3, lds, st, A);
     case 2: return gemv_dispatch<2>(g3, b3, lds, st, A);
+    // (Three and four rows come without the RMSNorm. Instances without its code were scheduled
+    // worse: 3 x 151936 x 4096 100 us against 88.)
     case 3: return gemv_dispatch<3>(g3, b3, lds, st, A);
     case 4: return gemv_dispatch<4>(g3, b3, lds, st, A);
     default: return hipErrorInvalidValue;
